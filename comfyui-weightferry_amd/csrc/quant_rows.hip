@@ -29,9 +29,14 @@
 // of the wave plays virtual threads l and l + 64. rstd = 1 / sqrt(var + eps) correctly rounded (the reference's
 // rsqrt.approx.f32 is an NVIDIA approximation).
 
+#include <algorithm>
+#include <type_traits>
+
 #include "wf_common.h"
 
 namespace wf {
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr float kAmaxClamp = 3.38953139e38f;
 
@@ -43,48 +48,70 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// RN(y / s) for the row's finite scale s, given rs = RN(1 / s). An infinite y (a rotation that overflowed)
-// gives y * rs = +-inf, which is the IEEE quotient; the correction step would turn it into NaN (inf - inf).
-__device__ __forceinline__ float div_rn(float y, float s, float rs) {
-    const float q = y * rs;
-    const float rem = __builtin_fmaf(-q, s, y);
-    const float r = __builtin_fmaf(rem, rs, q);
-    return __builtin_isinf(q) ? q : r;
+// the two bf16 values of a word as float32
+__device__ __forceinline__ float bf_lo(uint32_t u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float bf_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
+
+// LDS accesses of one wave run in the order they are issued, so a wave that exchanges values through its own LDS region
+// needs no wait: these fences only keep the compiler from moving one side's accesses past the other's.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ int8_t quant1(float y, float sb, float rsb) {
-    float v = __builtin_rintf(round_bf16(div_rn(round_bf16(y), sb, rsb)));
-    v = fminf(fmaxf(v, -128.0f), 127.0f);
-    return (int8_t)(int)v;
+// RN(y / s) for the row's finite scale s, given ns = -s and rs = RN(1 / s). HUGE rows (values past the amax clamp): an
+// infinite y (a rotation that overflowed) gives y * rs = +-inf, which is the IEEE quotient; the correction step would
+// turn it into NaN (inf - inf).
+template <bool HUGE_ROW>
+__device__ __forceinline__ float div_rn(float y, float ns, float rs) {
+    const float q = y * rs;
+    const float rem = __builtin_fmaf(q, ns, y);
+    const float r = __builtin_fmaf(rem, rs, q);
+    if constexpr (HUGE_ROW) return __builtin_isinf(q) ? q : r;
+    else return r;
+}
+
+// the int8 of a pair of bf16 values y (low byte of each word): rint(bf16(y / s)) clamped to [-128, 127], a NaN to -128.
+// The integer is read off the sum with 1.5 * 2^23, which rounds to nearest even as rint does.
+template <bool HUGE_ROW>
+__device__ __forceinline__ void quant2(uint32_t y, float ns, float rs, uint32_t& q0, uint32_t& q1) {
+    const uint32_t t = pack_bf16(div_rn<HUGE_ROW>(bf_lo(y), ns, rs), div_rn<HUGE_ROW>(bf_hi(y), ns, rs));
+    q0 = __float_as_uint(fminf(fmaxf(bf_lo(t), -128.0f), 127.0f) + 12582912.0f);
+    q1 = __float_as_uint(fminf(fmaxf(bf_hi(t), -128.0f), 127.0f) + 12582912.0f);
 }
 
 // the row's maximum over its W waves (W = 1: the wave's own); every lane of the W waves gets it. W > 1 needs the
 // whole workgroup to be one row (no wave leaves early), since it takes a workgroup barrier.
+// Calls in a loop alternate turn between 0 and 1: a wave may write its next maximum while another still reads these.
 template <int W>
-__device__ __forceinline__ float row_max(float wave_amax, int wave) {
+__device__ __forceinline__ float row_max(float wave_amax, int wave, int turn = 0) {
     if constexpr (W == 1) {
         return wave_amax;
     } else {
-        __shared__ float part[W];
-        if ((threadIdx.x & 63) == 0) part[wave] = wave_amax;
+        __shared__ float part[2][W];
+        if ((threadIdx.x & 63) == 0) part[turn][wave] = wave_amax;
         __syncthreads();
-        float m = part[0];
+        float m = part[turn][0];
 #pragma unroll
-        for (int i = 1; i < W; i++) m = fmaxf(m, part[i]);
+        for (int i = 1; i < W; i++) m = fmaxf(m, part[turn][i]);
         return m;
     }
 }
 
 struct RowScale {
-    float scale, sb, rsb;
+    float scale, nsb, rsb;     // the row's scale; minus its bf16 rounding, and that rounding's reciprocal
+    bool huge;                 // the row holds values past the amax clamp
 };
 
 __device__ __forceinline__ RowScale row_scale(float amax) {
     RowScale r;
+    r.huge = amax > kAmaxClamp;
     amax = fminf(amax, kAmaxClamp);
     r.scale = fmaxf(amax / 127.0f, 1.0e-30f);
-    r.sb = round_bf16(r.scale);
-    r.rsb = 1.0f / r.sb;
+    const float sb = round_bf16(r.scale);
+    r.nsb = -sb;
+    r.rsb = 1.0f / sb;
     return r;
 }
 
@@ -96,52 +123,90 @@ struct PreArgs {
     float eps;                // LNMOD
 };
 
+// Welford state of one virtual thread; its count is the same in every virtual thread at every step (K / 128 values
+// each, doubled by each merge), so the counts and what is derived from them are computed once, not per thread.
+struct Welford {
+    float m, s;
+};
+
 // PyTorch's cuWelfordCombine(dataB = own, dataA = other) as the reference restates it, with the contractions it
-// makes explicit (enhancers/fused_kernels.py:84-94)
-__device__ __forceinline__ void wcombine(float& m, float& s, float& c, float mo, float so, float co) {
-    const float delta = m - mo;
-    const float count = co + c;
-    const float coef = 1.0f / count;
-    const float na = co * coef, nb = c * coef;
-    const float mean = __builtin_fmaf(na, mo, nb * m);
-    const float sig = __builtin_fmaf((delta * delta) * co, nb, so + s);
-    m = mean; s = sig; c = count;
+// makes explicit (enhancers/fused_kernels.py:84-94); both sides hold co values, nab = co * (1 / (2 co))
+__device__ __forceinline__ void wcombine(Welford& w, float mo, float so, float co, float nab) {
+    const float delta = w.m - mo;
+    w.m = __builtin_fmaf(nab, mo, nab * w.m);
+    w.s = __builtin_fmaf((delta * delta) * co, nab, so + w.s);
 }
 
-// mean and sigma2 / K of one row (K % 512 == 0), every lane gets the result
+// lane i's value of x from lane i + O of its row of 16 (the lanes past the row's end get their own)
+template <int O>
+__device__ __forceinline__ float row_down(float x) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(x), __float_as_uint(x), 0x100 + O, 0xf, 0xf,
+                                                       false));
+}
+
+// 1 / c, correctly rounded, for the counts a virtual thread can reach (rows of up to 32768 values)
+struct Reciprocals {
+    float r[256];
+};
+static constexpr Reciprocals reciprocals() {
+    Reciprocals t{};
+    for (int c = 1; c <= 256; c++) t.r[c - 1] = 1.0f / (float)c;
+    return t;
+}
+__constant__ Reciprocals kRecip = reciprocals();
+
+// mean and sigma2 / K of one row (K % 512 == 0), every lane gets the result. The chain of updates is short; what it
+// costs is instructions, so the count's reciprocals come from a table (scalar loads) and the merges within rows of 16
+// lanes are DPP moves.
 __device__ __forceinline__ void ln_stats(const uint16_t* xr, int K, int lane, float& mu, float& var) {
-    float m[2] = {0.0f, 0.0f}, sg[2] = {0.0f, 0.0f}, c[2] = {0.0f, 0.0f};
-    for (int j = 0; j < (K >> 9); j++) {
+    Welford w[2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+    const int nj = K >> 9;
+#pragma unroll 4
+    for (int j = 0; j < nj; j++) {
+        uint2 u[2];
 #pragma unroll
-        for (int vt = 0; vt < 2; vt++) {
-            const int t = lane + 64 * vt;
-            const uint2 w = *reinterpret_cast<const uint2*>(xr + 4 * (t + 128 * j));
-            const float v4[4] = {bf16_bits_to_f32(w.x & 0xffffu), bf16_bits_to_f32(w.x >> 16),
-                                 bf16_bits_to_f32(w.y & 0xffffu), bf16_bits_to_f32(w.y >> 16)};
+        for (int vt = 0; vt < 2; vt++) u[vt] = *reinterpret_cast<const uint2*>(xr + 4 * (lane + 64 * vt + 128 * j));
 #pragma unroll
-            for (int ii = 0; ii < 4; ii++) {
-                const float delta = v4[ii] - m[vt];
-                c[vt] = c[vt] + 1.0f;
-                m[vt] = __builtin_fmaf(delta, 1.0f / c[vt], m[vt]);
-                sg[vt] = __builtin_fmaf(delta, v4[ii] - m[vt], sg[vt]);
+        for (int ii = 0; ii < 4; ii++) {
+            const float rc = kRecip.r[4 * j + ii];
+#pragma unroll
+            for (int vt = 0; vt < 2; vt++) {
+                const uint32_t p = ii < 2 ? u[vt].x : u[vt].y;
+                const float v = ii & 1 ? bf_hi(p) : bf_lo(p);
+                const float delta = v - w[vt].m;
+                w[vt].m = __builtin_fmaf(delta, rc, w[vt].m);
+                w[vt].s = __builtin_fmaf(delta, v - w[vt].m, w[vt].s);
             }
         }
     }
-    // within each 32-thread virtual warp: lane i < o merges lane i + o
+    // within each 32-thread virtual warp lane i < o merges lane i + o, o = 16, 8, 4, 2, 1 (the other lanes' results
+    // are not used)
+    // (every merge doubles the count, and rounding commutes with powers of two: co * RN(1 / (2 co)) is the same at
+    // each of them)
+    float co = (float)(4 * nj);
+    const float na = co * (0.5f * kRecip.r[4 * nj - 1]);
 #pragma unroll
-    for (int o = 16; o >= 1; o >>= 1) {
+    for (int vt = 0; vt < 2; vt++)
+        wcombine(w[vt], __shfl_down(w[vt].m, 16, 32), __shfl_down(w[vt].s, 16, 32), co, na);
+    auto merge = [&](auto o) {
+        constexpr int O = decltype(o)::value;
+        co = co + co;
 #pragma unroll
-        for (int vt = 0; vt < 2; vt++) {
-            const float mo = __shfl_down(m[vt], o, 32), so = __shfl_down(sg[vt], o, 32), co = __shfl_down(c[vt], o, 32);
-            if ((lane & 31) < o) wcombine(m[vt], sg[vt], c[vt], mo, so, co);
-        }
-    }
+        for (int vt = 0; vt < 2; vt++) wcombine(w[vt], row_down<O>(w[vt].m), row_down<O>(w[vt].s), co, na);
+    };
+    merge(std::integral_constant<int, 8>{});
+    merge(std::integral_constant<int, 4>{});
+    merge(std::integral_constant<int, 2>{});
+    merge(std::integral_constant<int, 1>{});
     // warps 2, 3 (lanes 0, 32 of the second virtual thread) into warps 0, 1; then warp 1 (lane 32) into warp 0
-    wcombine(m[0], sg[0], c[0], m[1], sg[1], c[1]);
-    const float mo = __shfl(m[0], 32, 64), so = __shfl(sg[0], 32, 64), co = __shfl(c[0], 32, 64);
-    wcombine(m[0], sg[0], c[0], mo, so, co);
-    mu = __shfl(m[0], 0, 64);
-    var = __shfl(sg[0], 0, 64) / (float)K;
+    co = co + co;
+    wcombine(w[0], w[1].m, w[1].s, co, na);
+    const float mo = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w[0].m), 32));
+    const float so = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w[0].s), 32));
+    co = co + co;
+    wcombine(w[0], mo, so, co, na);
+    mu = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(w[0].m)));
+    var = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(w[0].s))) / (float)K;
 }
 
 // ------------------------------------------------------------------------------------------------ plain rows
@@ -156,35 +221,54 @@ __global__ __launch_bounds__(256) void quant_plain(const uint16_t* __restrict__ 
     const uint4* xr = reinterpret_cast<const uint4*>(x + row * K);
     const int nchunks = K >> 3;
     uint4 v[CPL];
-    float amax = 0.0f;
+    // the maximum of the magnitudes' bits, two 16-bit halves at a time; with a NaN or an infinity among them the wave
+    // takes it in float32 instead (NaNs ignored), and the division that keeps infinite quotients
+    u16x2 mag = {0, 0};
 #pragma unroll
     for (int i = 0; i < CPL; i++) {
         const int c = (i * W + w) * 64 + lane;
         v[i] = c < nchunks ? xr[c] : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < CPL; i++) {
         const uint32_t u[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
 #pragma unroll
-        for (int h = 0; h < 4; h++) {
-            amax = fmaxf(amax, fabsf(bf16_bits_to_f32(u[h] & 0xffffu)));
-            amax = fmaxf(amax, fabsf(bf16_bits_to_f32(u[h] >> 16)));
+        for (int h = 0; h < 4; h++)
+            mag = __builtin_elementwise_max(mag, __builtin_bit_cast(u16x2, u[h] & 0x7fff7fffu));
+    }
+    const uint32_t top = max((uint32_t)mag[0], (uint32_t)mag[1]);
+    const bool special = __any(top >= 0x7f80u);
+    float amax = __uint_as_float(top << 16);
+    if (special) {
+        amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < CPL; i++) {
+            const uint32_t u[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+            for (int h = 0; h < 4; h++) amax = fmaxf(fmaxf(amax, fabsf(bf_lo(u[h]))), fabsf(bf_hi(u[h])));
         }
     }
     const RowScale rs = row_scale(row_max<W>(wave_max(amax), wave));
     if (lane == 0 && w == 0) xs[row] = rs.scale;
     uint2* qr = reinterpret_cast<uint2*>(xq + row * K);
+    auto store = [&](auto huge) {
 #pragma unroll
-    for (int i = 0; i < CPL; i++) {
-        const int c = (i * W + w) * 64 + lane;
-        if (c >= nchunks) continue;
-        const uint32_t u[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-        uint32_t b[2] = {0, 0};
+        for (int i = 0; i < CPL; i++) {
+            const int c = (i * W + w) * 64 + lane;
+            if (c >= nchunks) continue;
+            const uint32_t u[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+            uint32_t b[4];
 #pragma unroll
-        for (int h = 0; h < 4; h++) {
-            const uint32_t lo = (uint8_t)quant1(bf16_bits_to_f32(u[h] & 0xffffu), rs.sb, rs.rsb);
-            const uint32_t hi = (uint8_t)quant1(bf16_bits_to_f32(u[h] >> 16), rs.sb, rs.rsb);
-            b[h >> 1] |= (lo | (hi << 8)) << (16 * (h & 1));
+            for (int h = 0; h < 4; h++) {
+                uint32_t lo, hi;
+                quant2<decltype(huge)::value>(u[h], rs.nsb, rs.rsb, lo, hi);
+                b[h] = __builtin_amdgcn_perm(hi, lo, 0x0c0c0400u);     // (lo, hi) low bytes
+            }
+            qr[c] = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
         }
-        qr[c] = make_uint2(b[0], b[1]);
-    }
+    };
+    if (rs.huge || special) store(std::true_type{});
+    else store(std::false_type{});
 }
 
 // --------------------------------------------------------------------------------------------- ConvRot rows
@@ -197,119 +281,210 @@ __device__ __forceinline__ void h4(float& a, float& b, float& c, float& d) {
     a = y0; b = y1; c = y2; d = y3;
 }
 
-// LDS slot of element i (0..255) of group g of a wave's 4-group window: 17 floats per 16 elements (conflict-free
-// for both the contiguous and the stride-16 access)
-__device__ __forceinline__ int slot(int g, int i) { return g * 272 + i + (i >> 4); }
+// A wave's LDS window of 4 groups: 16 consecutive values of a group lie 20 floats apart, groups 336 apart, so that the
+// 16-byte writes of 16 consecutive values and the reads of 64 lanes' single values (value tl + 16 m of group gl) both
+// spread over all banks, and the writes stay 16-byte aligned.
+constexpr int kGroupFloats = 336, kRunFloats = 20;
+// the quantised bytes of a window, read back in 16-byte runs: groups 272 bytes apart (256 would put the four groups'
+// byte writes in the same banks)
+constexpr int kGroupBytes = 272;
+
+// GELU by table: the table's entries of the exponents [kGeluExp, kGeluExp + 24) -- magnitudes 2^-18 up to 64 -- are held
+// in LDS, both signs interleaved: entry 2 (|bits| - 128 kGeluExp) + sign. The few values outside come from the table.
+constexpr uint32_t kGeluExp = 109, kGeluEntries = 24 * 128, kGeluFirst = kGeluExp * 128;
 
 // W waves per row, NP passes of 4 groups (1024 values) per wave: K <= 1024 W NP, K % 256 == 0. Lane t of pass p
 // of wave w owns group 4 (p W + w) + t / 16, position tl = t % 16. W = 1: four rows per workgroup; W = 4: one.
+//
+// Bound by instruction issue, not by memory: about 20 vector instructions per value (10 of them the rotation's sums).
+// So the row's raw words of all passes load up front (their latency passes once), a rotated pass is kept as packed bf16
+// pairs (all the quotient uses; half the registers, more waves), the quotient's correction is two two-operand fmas, the
+// rounding to an integer one addition, and the LDS exchange is 16-byte writes with no waits. Measured on MI355X, before
+// and after, bit-identical: 16384 x 5120 67-69 and 51-53 us (4.9 TB/s), 4096 x 13824 53 and 39; GELU 5152 x 8192 48-49
+// and 40-42 (its table read from LDS instead of the L2), LayerNorm 5152 x 2048 24.1 and 18.5, 4096 x 8192 96 and 51
+// (its statistics had an IEEE division per value); scale-and-shift 4096 x 5120 24.8 and 24.2.
 template <int NP, int PRE, int W>
 __global__ __launch_bounds__(256) void quant_convrot(const uint16_t* __restrict__ x, int64_t M, int K,
                                                      int8_t* __restrict__ xq, float* __restrict__ xs, PreArgs pa) {
-    __shared__ float stage[4][4 * 272];          // per wave: one 4-group window
-    __shared__ uint32_t qbytes[4][256];          // per wave: the 1024 int8 values of one pass, 4 bytes a word
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, w = wave % W;
-    const int64_t row = (int64_t)blockIdx.x * (4 / W) + wave / W;
-    if (W == 1 && row >= M) return;              // whole waves leave together; W = 1 takes no workgroup barrier
+    __shared__ __align__(16) float stage[4][4 * kGroupFloats];      // per wave: one 4-group window
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, w = wave % W;
+    int64_t row = (int64_t)blockIdx.x * (4 / W) + wave / W;
     const int G = K >> 8;                        // groups in the row
     const int gl = lane >> 4, tl = lane & 15;
-    float* st = stage[wave];
-    float y[NP][16];
-    float amax = 0.0f;
-    float mu = 0.0f, rstd = 0.0f;
-    const int64_t grp = PRE >= 2 ? row / pa.rows_per_group : 0;
-    if constexpr (PRE == 3) {
-        float var;
-        ln_stats(x + row * K, K, lane, mu, var);
-        rstd = (float)(1.0 / __builtin_sqrt((double)(var + pa.eps)));
-    }
-#pragma unroll
-    for (int p = 0; p < NP; p++) {
-        const int g = 4 * (p * W + w) + gl;
-        const bool live = g < G;
-        // 16 consecutive values [16 tl, 16 tl + 16) of group g: digits k0 (stride 1) and k1 (stride 4)
-        float v[16];
-        if (live) {
-            const uint4* src = reinterpret_cast<const uint4*>(x + row * K + g * 256 + 16 * tl);
-            const uint4 a = src[0], b = src[1];
-            const uint32_t u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-            for (int h = 0; h < 8; h++) {
-                v[2 * h] = bf16_bits_to_f32(u[h] & 0xffffu);
-                v[2 * h + 1] = bf16_bits_to_f32(u[h] >> 16);
-            }
-            if constexpr (PRE == 1) {
-#pragma unroll
-                for (int h = 0; h < 8; h++) {
-                    v[2 * h] = bf16_bits_to_f32(pa.s[u[h] & 0xffffu]);
-                    v[2 * h + 1] = bf16_bits_to_f32(pa.s[u[h] >> 16]);
-                }
-            } else if constexpr (PRE >= 2) {
-                const int64_t o = grp * K + g * 256 + 16 * tl;
-                const uint4* sp = reinterpret_cast<const uint4*>(pa.s + o);
-                const uint4* hp = reinterpret_cast<const uint4*>(pa.h + o);
-                const uint4 s0 = sp[0], s1 = sp[1], h0 = hp[0], h1 = hp[1];
-                const uint32_t sw[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-                const uint32_t hw[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const float sc = bf16_bits_to_f32(i & 1 ? sw[i >> 1] >> 16 : sw[i >> 1] & 0xffffu);
-                    const float sh = bf16_bits_to_f32(i & 1 ? hw[i >> 1] >> 16 : hw[i >> 1] & 0xffffu);
-                    float t = v[i];
-                    if constexpr (PRE == 3) t = round_bf16((t - mu) * rstd);
-                    v[i] = round_bf16(round_bf16(t * sc) + sh);
-                }
+    const uint16_t* gelu = nullptr;
+    if constexpr (PRE == 1) {
+        __shared__ __align__(16) uint16_t tab[2 * kGeluEntries];
+        if ((reinterpret_cast<uintptr_t>(pa.s) & 15) == 0) {
+            for (int i = threadIdx.x; i < (int)kGeluEntries / 8; i += 256) {
+                const uint4 a = reinterpret_cast<const uint4*>(pa.s + kGeluFirst)[i];
+                const uint4 b = reinterpret_cast<const uint4*>(pa.s + 0x8000u + kGeluFirst)[i];
+                uint4* t = reinterpret_cast<uint4*>(tab + 16 * i);
+                auto even = [](uint32_t u, uint32_t v) { return __builtin_amdgcn_perm(v, u, 0x05040100u); };
+                auto odd = [](uint32_t u, uint32_t v) { return __builtin_amdgcn_perm(v, u, 0x07060302u); };
+                t[0] = make_uint4(even(a.x, b.x), odd(a.x, b.x), even(a.y, b.y), odd(a.y, b.y));
+                t[1] = make_uint4(even(a.z, b.z), odd(a.z, b.z), even(a.w, b.w), odd(a.w, b.w));
             }
         } else {
-#pragma unroll
-            for (int i = 0; i < 16; i++) v[i] = 0.0f;
+            for (int i = threadIdx.x; i < (int)kGeluEntries; i += 256) {
+                tab[2 * i] = pa.s[kGeluFirst + i];
+                tab[2 * i + 1] = pa.s[0x8000u + kGeluFirst + i];
+            }
         }
-#pragma unroll
-        for (int q = 0; q < 4; q++) h4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);   // stride 1
-#pragma unroll
-        for (int q = 0; q < 4; q++) h4(v[q], v[q + 4], v[q + 8], v[q + 12]);                  // stride 4
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int i = 0; i < 16; i++) st[slot(gl, 16 * tl + i)] = v[i];
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_s_waitcnt(0);           // LDS writes of this wave done before the reads below
-        __builtin_amdgcn_wave_barrier();
-        // now the 16 values i = tl + 16 m (m = k2 + 4 k3) of group g
-#pragma unroll
-        for (int m = 0; m < 16; m++) v[m] = st[slot(gl, tl + 16 * m)];
-#pragma unroll
-        for (int q = 0; q < 4; q++) h4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);   // stride 16
-#pragma unroll
-        for (int q = 0; q < 4; q++) h4(v[q], v[q + 4], v[q + 8], v[q + 12]);                  // stride 64
-#pragma unroll
-        for (int m = 0; m < 16; m++) {
-            y[p][m] = v[m] * 0.0625f;
-            if (live) amax = fmaxf(amax, fabsf(y[p][m]));
-        }
-        __builtin_amdgcn_wave_barrier();
+        gelu = tab;
+        __syncthreads();
     }
-    const RowScale rs = row_scale(row_max<W>(wave_max(amax), wave));
-    if (lane == 0 && w == 0) xs[row] = rs.scale;
-    // per pass: quantise into the wave's LDS words at the bytes' row positions, then store the pass's 1024 bytes
-    // (four whole groups, contiguous in the row) with one 16-byte store per lane
-    uint8_t* qb = reinterpret_cast<uint8_t*>(qbytes[wave]);
-    const uint4* qs = reinterpret_cast<const uint4*>(qbytes[wave]);
-    uint4* dst = reinterpret_cast<uint4*>(xq + row * K);
+    if (W == 1 && row >= M) return;              // whole waves leave together; W = 1 takes no further workgroup barrier
+    float* st = stage[wave];
+    // 16 consecutive values [16 tl, 16 tl + 16) of this lane's group of pass p
+    auto at = [&](int p) { return 256 * (4 * (p * W + w) + gl) + 16 * tl; };
+    auto live = [&](int p) { return 4 * (p * W + w) + gl < G; };
+    uint4 raw[NP][2];
+    auto load_row = [&](int64_t r) {
 #pragma unroll
-    for (int p = 0; p < NP; p++) {
-        const int g0 = 4 * (p * W + w);
-        if (g0 >= G) break;                      // the same for the whole wave
-        if (g0 + gl < G) {
-#pragma unroll
-            for (int m = 0; m < 16; m++) qb[gl * 256 + tl + 16 * m] = (uint8_t)quant1(y[p][m], rs.sb, rs.rsb);
+        for (int p = 0; p < NP; p++) {
+            raw[p][0] = raw[p][1] = make_uint4(0, 0, 0, 0);
+            if (live(p)) {
+                const uint4* src = reinterpret_cast<const uint4*>(x + r * K + at(p));
+                raw[p][0] = src[0];
+                raw[p][1] = src[1];
+            }
         }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        if (g0 + (lane >> 4) < G) dst[g0 * 16 + lane] = qs[lane];
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_s_waitcnt(0);           // the pass's LDS reads done before the next pass writes
-        __builtin_amdgcn_wave_barrier();
+    };
+    // (with more passes the next row's words would cost waves)
+    constexpr bool AHEAD = PRE == 1 && NP <= 3;
+    load_row(row);
+    // scale and shift of a pass, loaded a pass ahead
+    uint4 sh[2][4];
+    auto load_mod = [&](const uint16_t* s, const uint16_t* h, int p) {
+        if (p < NP && live(p)) {
+            const uint4* sp = reinterpret_cast<const uint4*>(s + at(p));
+            const uint4* hp = reinterpret_cast<const uint4*>(h + at(p));
+            sh[p & 1][0] = sp[0];
+            sh[p & 1][1] = sp[1];
+            sh[p & 1][2] = hp[0];
+            sh[p & 1][3] = hp[1];
+        }
+    };
+    // GELU: the grid holds a few workgroups per CU, each taking every gridDim.x-th row (or four rows), so that the table
+    // is loaded that often only; the next row's words load while this one's are quantised. Otherwise one turn.
+    for (int turn = 0;; turn ^= 1) {
+        float mu = 0.0f, rstd = 0.0f;
+        const uint16_t *sr = nullptr, *hr = nullptr;
+        if constexpr (PRE >= 2) {
+            // (32-bit division where it fits: the 64-bit one is a long sequence)
+            const int64_t grp = M < (1LL << 31) && pa.rows_per_group < (1LL << 31)
+                                    ? (int64_t)((uint32_t)row / (uint32_t)pa.rows_per_group)
+                                    : row / pa.rows_per_group;
+            sr = pa.s + grp * K;
+            hr = pa.h + grp * K;
+            load_mod(sr, hr, 0);
+        }
+        if constexpr (PRE == 3) {
+            float var;
+            ln_stats(x + row * K, K, lane, mu, var);
+            rstd = (float)(1.0 / __builtin_sqrt((double)(var + pa.eps)));
+        }
+        uint32_t y[NP][8];                           // the rotated values as bf16 pairs (values m, m + 1)
+        float amax = 0.0f;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            uint32_t u[8] = {raw[p][0].x, raw[p][0].y, raw[p][0].z, raw[p][0].w,
+                             raw[p][1].x, raw[p][1].y, raw[p][1].z, raw[p][1].w};
+            if constexpr (PRE == 1) {
+                if (live(p)) {
+                    // |bits| of the pairs' members; all 16 in the LDS part of the table, or value by value
+                    uint32_t lo = 0xffffffffu, hi = 0;
+#pragma unroll
+                    for (int h = 0; h < 8; h++) {
+                        const uint32_t a = u[h] & 0x7fffu, b = (u[h] >> 16) & 0x7fffu;
+                        lo = min(lo, min(a, b));
+                        hi = max(hi, max(a, b));
+                    }
+                    auto slot = [&](uint32_t b) { return 2u * (b & 0x7fffu) + (b >> 15) - 2u * kGeluFirst; };
+                    if (lo >= kGeluFirst && hi < kGeluFirst + kGeluEntries) {
+#pragma unroll
+                        for (int h = 0; h < 8; h++)
+                            u[h] = gelu[slot(u[h] & 0xffffu)] | ((uint32_t)gelu[slot(u[h] >> 16)] << 16);
+                    } else {
+#pragma unroll
+                        for (int h = 0; h < 8; h++)
+                            u[h] = pa.s[u[h] & 0xffffu] | ((uint32_t)pa.s[u[h] >> 16] << 16);
+                    }
+                }
+            } else if constexpr (PRE >= 2) {
+                load_mod(sr, hr, p + 1);
+                if (live(p)) {
+                    const uint4 s0 = sh[p & 1][0], s1 = sh[p & 1][1], h0 = sh[p & 1][2], h1 = sh[p & 1][3];
+                    const uint32_t sw[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+                    const uint32_t hw[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+#pragma unroll
+                    for (int h = 0; h < 8; h++) {
+                        if constexpr (PRE == 3) u[h] = pack_bf16((bf_lo(u[h]) - mu) * rstd, (bf_hi(u[h]) - mu) * rstd);
+                        u[h] = pack_bf16(bf_lo(u[h]) * bf_lo(sw[h]), bf_hi(u[h]) * bf_hi(sw[h]));
+                        u[h] = pack_bf16(bf_lo(u[h]) + bf_lo(hw[h]), bf_hi(u[h]) + bf_hi(hw[h]));
+                    }
+                }
+            }
+            float v[16];
+#pragma unroll
+            for (int h = 0; h < 8; h++) {
+                v[2 * h] = bf_lo(u[h]);
+                v[2 * h + 1] = bf_hi(u[h]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) h4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);   // stride 1
+#pragma unroll
+            for (int q = 0; q < 4; q++) h4(v[q], v[q + 4], v[q + 8], v[q + 12]);                  // stride 4
+            wave_lds_order();
+            float4* run = reinterpret_cast<float4*>(st + gl * kGroupFloats + tl * kRunFloats);
+#pragma unroll
+            for (int q = 0; q < 4; q++) run[q] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+            wave_lds_order();
+            // now the 16 values i = tl + 16 m (m = k2 + 4 k3) of the group
+#pragma unroll
+            for (int m = 0; m < 16; m++) v[m] = st[gl * kGroupFloats + m * kRunFloats + tl];
+#pragma unroll
+            for (int q = 0; q < 4; q++) h4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);   // stride 16
+#pragma unroll
+            for (int q = 0; q < 4; q++) h4(v[q], v[q + 4], v[q + 8], v[q + 12]);                  // stride 64
+#pragma unroll
+            for (int h = 0; h < 8; h++) {
+                const float a = v[2 * h] * 0.0625f, b = v[2 * h + 1] * 0.0625f;
+                amax = fmaxf(fmaxf(amax, fabsf(a)), fabsf(b));      // (a lane past the row's end holds zeros)
+                y[p][h] = pack_bf16(a, b);
+            }
+        }
+        const int64_t next = row + (int64_t)gridDim.x * (4 / W);
+        if constexpr (AHEAD) {
+            if (next < M) load_row(next);
+        }
+        const RowScale rs = row_scale(row_max<W>(wave_max(amax), wave, turn));
+        if (lane == 0 && w == 0) xs[row] = rs.scale;
+        // per pass: quantise into the wave's LDS window at the bytes' row positions, then store the pass's 1024 bytes
+        // (four whole groups, contiguous in the row) with one 16-byte store per lane
+        uint8_t* qb = reinterpret_cast<uint8_t*>(st) + gl * kGroupBytes;
+        uint8_t* dst = reinterpret_cast<uint8_t*>(xq + row * K);
+        auto store = [&](auto huge) {
+#pragma unroll
+            for (int p = 0; p < NP; p++) {
+                if (4 * (p * W + w) >= G) break;     // the same for the whole wave
+                wave_lds_order();
+#pragma unroll
+                for (int h = 0; h < 8; h++) {
+                    uint32_t q0, q1;
+                    quant2<decltype(huge)::value>(y[p][h], rs.nsb, rs.rsb, q0, q1);
+                    qb[tl + 32 * h] = (uint8_t)q0;
+                    qb[tl + 32 * h + 16] = (uint8_t)q1;
+                }
+                wave_lds_order();
+                if (live(p)) *reinterpret_cast<uint4*>(dst + at(p)) = *reinterpret_cast<const uint4*>(qb + 16 * tl);
+            }
+        };
+        if (rs.huge) store(std::true_type{});
+        else store(std::false_type{});
+        if (PRE != 1 || next >= M) break;
+        row = next;
+        if constexpr (!AHEAD) load_row(row);
     }
 }
 
@@ -341,7 +516,9 @@ static void launch_plain_rows(const uint16_t* x, int64_t M, int K, int8_t* xq, f
 template <int NP, int PRE, int W>
 static void launch_convrot_pre(const uint16_t* x, int64_t M, int K, int8_t* xq, float* xs, const PreArgs& pa,
                                hipStream_t s) {
-    quant_convrot<NP, PRE, W><<<dim3((unsigned)((M + 4 / W - 1) / (4 / W))), 256, 0, s>>>(x, M, K, xq, xs, pa);
+    int64_t grid = (M + 4 / W - 1) / (4 / W);
+    if (PRE == 1) grid = std::min<int64_t>(grid, 4 * 256);      // four workgroups' LDS fit a CU
+    quant_convrot<NP, PRE, W><<<dim3((unsigned)grid), 256, 0, s>>>(x, M, K, xq, xs, pa);
 }
 
 template <int PRE>

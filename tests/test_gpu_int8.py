@@ -246,6 +246,26 @@ def test_quant_rows_pre_against_oracle(native, pre, K, groups, rows):
     assert bad.size == 0, bad[:8].tolist()
 
 
+@pytest.mark.parametrize("M,K,offset", [(4099, 256, 0), (4099, 3072, 1), (1027, 6400, 0)])
+def test_gelu_rows_over_several_turns(native, M, K, offset):
+    # more rows than the grid takes at once (4096 in single waves, 1024 in whole workgroups), and values outside the part
+    # of the table the kernel holds in LDS (zeros, tiny, large): one in each row, then whole rows of them; the table
+    # 16-byte aligned and not
+    g = torch.Generator().manual_seed(M + K)
+    x = (torch.randn((M, K), generator=g) * 1.5).to(torch.bfloat16)
+    odd = torch.tensor([0.0, -0.0, 1e-6, -3e-6, 64.0, -64.0, 3e4, -1e-38, 63.75, 3.9e-6]).to(torch.bfloat16)
+    x[torch.arange(M), torch.arange(M) % K] = odd[torch.arange(M) % 10]
+    x[5] = odd[torch.arange(K) % 10]
+    x[M - 1] = 0.0
+    table, tbits = _gelu_table_bits()
+    held = torch.empty(65536 + 8, dtype=torch.bfloat16, device="cuda")[offset:offset + 65536]
+    held.copy_(table)
+    xq, xs = gpu_quant_pre(native, x.cuda(), 1, held)
+    rq, rs = lib.quant_rows_pre(_bits(x), 1, tbits)
+    assert np.array_equal(xs.cpu().numpy().view(np.uint32), rs.view(np.uint32))
+    assert np.array_equal(xq.cpu().numpy(), rq)
+
+
 @pytest.mark.parametrize("kind,K", [("mod", 5120), ("gelu", 5120), ("lnmod", 4096), ("mod", 13824),
                                     ("gelu", 20480), ("lnmod", 8192)])
 def test_pending_input_quantised_with_its_operation(native, kind, K):
