@@ -689,6 +689,234 @@ static void launch_all(int mid_dt, int out_dt, int qtype, const uint8_t* src, vo
     else launch_mid<WF_F32, ADD>(out_dt, qtype, src, out, nblocks, diff, sa, s);
 }
 
+// ------------------------------------------------------------------------------------------ LoRA in one kernel
+// out = OUT(w + OUT(diff * sa)), diff = up @ down in float32: wf_dequant_add with the difference computed where it is
+// added. The float32 product written to HBM and read back (64 MiB each way for an 8192 x 2048 weight) and the float32
+// copies of both factors are what bounded the chain before; here a workgroup keeps the difference of its 32 x 256
+// tile in LDS. The product is v_mfma_f32_32x32x2_f32, one chain per value in the order of the rank, the factors
+// widened exactly from float16 / bfloat16: nothing is rounded that a float32 matrix product would not round.
+// MFMA rows are weight columns, so a lane's 16 + 16 sums of two tiles (columns 2a and 2a + 1) are runs of 8 columns of
+// one weight row and leave as two 16-byte LDS writes; rows are 260 floats apart (65 slots of 16 bytes: conflict-free).
+// 33 KiB of LDS: four workgroups a CU, whose loads, products and stores overlap.
+// Measured on MI355X, bf16 factors on the device, against the casts, torch.mm and wf_dequant_add (us): 8192 x 2048
+// Q5_1 at rank 4 / 32 / 128 15.2 / 21.9 / 53.9 against 44.6 / 47.2 / 65.2; 5120 x 5120 Q4_K 21.0 / 33.0 / 86.3 against
+// 66.3 / 72.9 / 145.6. About 11 us of memory traffic and 0.34 us per rank at 8192 x 2048, the float32 matrix unit's
+// time; at rank 256 the library's larger tiles are as fast (98.0 against 93.7), so the kernel stops before it.
+constexpr int kLoraRankMax = 192;
+constexpr int kLoraRows = 32, kLoraCols = 256, kLoraPitch = 260;
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+struct LoraArgs {
+    const void* up;       // [n_out, rank] of dtype up_dt
+    const void* down;     // [rank, n_in] of dtype down_dt
+    int up_dt, down_dt, rank, up_vec;    // up_vec: up rows are whole 16-byte runs of 8 two-byte values
+    int64_t n_out;
+    uint32_t n_in;
+    float sa;
+};
+
+__device__ __forceinline__ float widen(uint32_t bits16, int dt) {
+    return dt == WF_BF16 ? __uint_as_float(bits16 << 16) : f16_bits_to_f32(bits16);
+}
+
+// the tile's float32 difference at e0 + shift (e0 relative to the first value of the tile's first row)
+struct AddTile {
+    void* out;
+    const float* tile;
+    int shift;
+    float sa;
+    template <int OUT>
+    __device__ __forceinline__ void put(int64_t e0, const float (&v)[8]) const {
+        float w[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) w[i] = round_to<OUT>(v[i]);
+        add_scaled<OUT>(w, tile + ((int)e0 + shift), sa);
+        store8<OUT>(out, e0, w);
+    }
+    template <int OUT>
+    __device__ __forceinline__ void puth(int64_t e0, const h2 (&v)[4]) const {
+        float f[8];
+#pragma unroll
+        for (int i = 0; i < 4; i++) { f[2 * i] = (float)v[i][0]; f[2 * i + 1] = (float)v[i][1]; }
+        put<OUT>(e0, f);
+    }
+};
+
+// values already in the output, for the LoRAs after the first: a lane-item is 8 of them
+template <int OUT_>
+struct Held {
+    static constexpr int LANES_PER_BLOCK = 1, PER = 8, OUT_BYTES = OUT_ == WF_F32 ? 4 : 2, TS = 8 * OUT_BYTES;
+    struct Raw { uint4 a, b; };
+    static __device__ __forceinline__ Raw load(const uint8_t* src, uint32_t t) {
+        const uint4* p = reinterpret_cast<const uint4*>(src + (int64_t)t * TS);
+        Raw r;
+        r.a = p[0];
+        if constexpr (OUT_ == WF_F32) r.b = p[1];
+        return r;
+    }
+    template <class S>
+    static __device__ __forceinline__ void emit(const S& o, uint32_t t, const Raw& r) {
+        float v[8];
+        if constexpr (OUT_ == WF_F32) {
+            const uint32_t u[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = __uint_as_float(u[i]);
+        } else {
+            const uint32_t u[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) { v[2 * i] = widen(u[i] & 0xffffu, OUT_); v[2 * i + 1] = widen(u[i] >> 16, OUT_); }
+        }
+        o.template put<OUT_>(8 * (int64_t)t, v);
+    }
+};
+
+// acc0 / acc1 += a wave's 32 rows x 64 columns of up @ down, from row row0 (rows of them exist) and column c0. Lane
+// (ln, lk) holds columns c0 + 2 ln and + 1 of down's row k and up's row ln, k = 2 s + lk of the MFMA step s. The next
+// eight ranks' loads are in flight under this eight's MFMAs, and a value is widened only where it is used: widened
+// behind its load, each load was waited for in turn (8192 x 2048 of rank 64: 44 us). Indexes are clamped instead of
+// branched on: rows and columns past the end give sums that are not used, ranks past the end are zeros in both.
+template <bool DF32, bool UVEC>
+__device__ __forceinline__ void lora_product(const LoraArgs& a, int64_t row0, int rows, uint32_t c0, int ln, int lk,
+                                             f32x16& acc0, f32x16& acc1) {
+    struct Chunk { uint32_t d0[4], d1[4], u[4]; };
+    const uint32_t c = min(c0 + 2 * ln, a.n_in - 2);                  // n_in is even
+    const int64_t n = row0 + min(ln, rows - 1);
+    auto load = [&](int k0) {
+        Chunk q;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int64_t at = (int64_t)min(k0 + 2 * s + lk, a.rank - 1) * a.n_in + c;
+            if constexpr (DF32) {
+                const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const float*>(a.down) + at);
+                q.d0[s] = v.x;
+                q.d1[s] = v.y;
+            } else {
+                q.d0[s] = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.down) + at);
+            }
+        }
+        if constexpr (UVEC) {
+            const uint4 v = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.up) + n * a.rank +
+                                                            min(k0, a.rank - 8));
+            q.u[0] = v.x; q.u[1] = v.y; q.u[2] = v.z; q.u[3] = v.w;
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const int64_t at = n * a.rank + min(k0 + 2 * s + lk, a.rank - 1);
+                q.u[s] = a.up_dt == WF_F32 ? static_cast<const uint32_t*>(a.up)[at] : static_cast<const uint16_t*>(a.up)[at];
+            }
+        }
+        return q;
+    };
+    Chunk q = load(0);
+    for (int k0 = 0; k0 < a.rank; k0 += 8) {
+        const Chunk nx = load(k0 + 8);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            float d0, d1, u;
+            if constexpr (DF32) {
+                d0 = __uint_as_float(q.d0[s]);
+                d1 = __uint_as_float(q.d1[s]);
+            } else {
+                d0 = widen(q.d0[s] & 0xffffu, a.down_dt);
+                d1 = widen(q.d0[s] >> 16, a.down_dt);
+            }
+            if constexpr (UVEC) u = widen(lk ? q.u[s] >> 16 : q.u[s] & 0xffffu, a.up_dt);
+            else u = a.up_dt == WF_F32 ? __uint_as_float(q.u[s]) : widen(q.u[s], a.up_dt);
+            if constexpr (!UVEC) {                                    // (UVEC: the rank is a multiple of 8)
+                const bool past = k0 + 2 * s + lk >= a.rank;
+                d0 = past ? 0.0f : d0;
+                d1 = past ? 0.0f : d1;
+                u = past ? 0.0f : u;
+            }
+            acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(d0, u, acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(d1, u, acc1, 0, 0, 0);
+        }
+        q = nx;
+    }
+}
+
+template <typename F>
+__global__ __launch_bounds__(256) void deq_lora(const uint8_t* src, void* out, LoraArgs a) {
+    constexpr int LPR = kLoraCols / F::PER * F::LANES_PER_BLOCK;      // lane-items per tile row
+    constexpr int ITEMS = kLoraRows * LPR / 256;                      // per thread
+    constexpr int BPT = kLoraCols / F::PER;                           // blocks per tile row
+    __shared__ float tile[kLoraRows * kLoraPitch];
+    const uint32_t ntc = (a.n_in + kLoraCols - 1) / kLoraCols;
+    const uint32_t tr = __builtin_amdgcn_readfirstlane(blockIdx.x / ntc);
+    const uint32_t tc = __builtin_amdgcn_readfirstlane(blockIdx.x - tr * ntc);
+    const int64_t row0 = (int64_t)tr * kLoraRows;
+    const uint32_t col0 = tc * kLoraCols, bpr = a.n_in / F::PER;
+    const int rows = (int)min((int64_t)kLoraRows, a.n_out - row0);
+    const uint8_t* tsrc = src + row0 * bpr * F::TS;
+    void* tout = static_cast<char*>(out) + row0 * a.n_in * F::OUT_BYTES;
+    // this thread's lane-items: their blocks' bytes leave first and land under the product
+    typename F::Raw raw[ITEMS];
+    uint32_t item[ITEMS];
+    bool in[ITEMS];
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++) {
+        const uint32_t i = threadIdx.x + 256u * u, r = i / LPR, j = i % LPR;
+        in[u] = (int)r < rows && tc * BPT + j / F::LANES_PER_BLOCK < bpr;
+        item[u] = (r * bpr + tc * BPT) * F::LANES_PER_BLOCK + j;
+        if (in[u]) raw[u] = F::load(tsrc, item[u]);
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ln = lane & 31, lk = lane >> 5;
+    f32x16 acc0, acc1;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc0[e] = acc1[e] = 0.0f;
+    if (a.down_dt == WF_F32) {
+        if (a.up_vec) lora_product<true, true>(a, row0, rows, col0 + 64 * wave, ln, lk, acc0, acc1);
+        else lora_product<true, false>(a, row0, rows, col0 + 64 * wave, ln, lk, acc0, acc1);
+    } else {
+        if (a.up_vec) lora_product<false, true>(a, row0, rows, col0 + 64 * wave, ln, lk, acc0, acc1);
+        else lora_product<false, false>(a, row0, rows, col0 + 64 * wave, ln, lk, acc0, acc1);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        float4* p = reinterpret_cast<float4*>(tile + ln * kLoraPitch + 64 * wave + 16 * g + 8 * lk);
+        p[0] = make_float4(acc0[4 * g], acc1[4 * g], acc0[4 * g + 1], acc1[4 * g + 1]);
+        p[1] = make_float4(acc0[4 * g + 2], acc1[4 * g + 2], acc0[4 * g + 3], acc1[4 * g + 3]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++) {
+        if (!in[u]) continue;
+        const int r = (int)((threadIdx.x + 256u * u) / LPR);
+        F::emit(AddTile{tout, tile, r * (kLoraPitch - (int)a.n_in) - (int)col0, a.sa}, item[u], raw[u]);
+    }
+}
+
+template <typename F>
+static void launch_lora(const uint8_t* src, void* out, const LoraArgs& a, hipStream_t s) {
+    const int64_t tiles = (a.n_out + kLoraRows - 1) / kLoraRows * ((a.n_in + kLoraCols - 1) / kLoraCols);
+    deq_lora<F><<<dim3((unsigned)tiles), 256, 0, s>>>(src, out, a);
+}
+
+template <int MID, int OUT>
+static void lora_fmt(int qtype, const uint8_t* src, void* out, const LoraArgs& a, hipStream_t s) {
+    switch (qtype) {
+    case 8: launch_lora<Q8_0<MID, OUT>>(src, out, a, s); break;
+    case 12: launch_lora<Q45_K<12, MID, OUT>>(src, out, a, s); break;
+    case 13: launch_lora<Q45_K<13, MID, OUT>>(src, out, a, s); break;
+    case 14: launch_lora<Q6_K<MID, OUT>>(src, out, a, s); break;
+    case 2: launch_lora<Legacy<2, MID, OUT>>(src, out, a, s); break;
+    case 3: launch_lora<Legacy<3, MID, OUT>>(src, out, a, s); break;
+    case 6: launch_lora<Legacy<6, MID, OUT>>(src, out, a, s); break;
+    case 7: launch_lora<Legacy<7, MID, OUT>>(src, out, a, s); break;
+    case 10: launch_lora<Q2_K<MID, OUT>>(src, out, a, s); break;
+    case 11: launch_lora<Q3_K<MID, OUT>>(src, out, a, s); break;
+    default: break;
+    }
+}
+
+template <int MID>
+static void lora_mid(int out_dt, int qtype, const uint8_t* src, void* out, const LoraArgs& a, hipStream_t s) {
+    if (out_dt == WF_F16) lora_fmt<MID, WF_F16>(qtype, src, out, a, s);
+    else if (out_dt == WF_BF16) lora_fmt<MID, WF_BF16>(qtype, src, out, a, s);
+    else lora_fmt<MID, WF_F32>(qtype, src, out, a, s);
+}
+
 // bytes per block and values per block of a supported GGML type (0 when unsupported)
 int block_bytes(int qtype, int* per) {
     switch (qtype) {
@@ -781,5 +1009,53 @@ extern "C" int wf_dequant_add(const void* src, int64_t src_bytes, int qtype, int
     if (!aligned(diff, 16)) { set_error("wf_dequant_add: diff must be 16-byte aligned"); return WF_EUNSUPPORTED; }
     launch_all<true>(mid_dt, out_dt, qtype, static_cast<const uint8_t*>(src), out, nblocks, diff, scale, s);
     WF_LAUNCH_CHECK("wf_dequant_add launch");
+    return WF_OK;
+}
+
+extern "C" int wf_dequant_lora(const void* src, int64_t src_bytes, int qtype, int mid_dt, int out_dt, const void* up,
+                               int up_dt, const void* down, int down_dt, int64_t rank, float scale, void* out,
+                               int64_t n_out, int64_t n_in, void* stream) {
+    using namespace wf;
+    if (n_out < 0 || n_in < 0 || rank < 0) {
+        set_error("wf_dequant_lora: %lld x %lld, rank %lld", (long long)n_out, (long long)n_in, (long long)rank);
+        return WF_EINVAL;
+    }
+    // 32-bit lane offsets inside a tile's 32 rows, and a grid of at most 2^31 - 1 workgroups
+    if (n_in > (1 << 24) || n_out > (1LL << 30) || rank < 1 || rank > kLoraRankMax ||
+        (n_out / kLoraRows + 1) * (n_in / kLoraCols + 1) >= (1LL << 31)) {
+        set_error("wf_dequant_lora: %lld x %lld of rank %lld is beyond the kernel's sizes", (long long)n_out,
+                  (long long)n_in, (long long)rank);
+        return WF_EUNSUPPORTED;
+    }
+    if (out_dt < 0 || out_dt > 2 || up_dt < 0 || up_dt > 2 || down_dt < 0 || down_dt > 2) {
+        set_error("wf_dequant_lora: dtype codes %d / %d / %d", out_dt, up_dt, down_dt);
+        return WF_EUNSUPPORTED;
+    }
+    int per = 8;
+    if (src) {
+        int64_t nblocks = 0;
+        const int rc = check_blocks("wf_dequant_lora", src, src_bytes, qtype, mid_dt, out_dt, out, n_out * n_in, &nblocks);
+        if (rc != WF_OK) return rc;
+        block_bytes(qtype, &per);
+    }
+    if (n_in % per) { set_error("wf_dequant_lora: rows of %lld values are not whole blocks", (long long)n_in); return WF_EUNSUPPORTED; }
+    if (n_out == 0 || n_in == 0) return WF_OK;
+    if (!out || !up || !down) { set_error("wf_dequant_lora: null pointer"); return WF_EINVAL; }
+    if (!aligned(out, 16) || !aligned(up, up_dt == WF_F32 ? 4 : 2) || !aligned(down, down_dt == WF_F32 ? 8 : 4)) {
+        set_error("wf_dequant_lora: out 16-byte aligned, up on its values, down on pairs of its values");
+        return WF_EUNSUPPORTED;
+    }
+    const LoraArgs a{up, down, up_dt, down_dt, (int)rank, up_dt != WF_F32 && rank % 8 == 0 && aligned(up, 16), n_out,
+                     (uint32_t)n_in, scale};
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const uint8_t* b = static_cast<const uint8_t*>(src ? src : out);
+    if (!src) {
+        if (out_dt == WF_F16) launch_lora<Held<WF_F16>>(b, out, a, s);
+        else if (out_dt == WF_BF16) launch_lora<Held<WF_BF16>>(b, out, a, s);
+        else launch_lora<Held<WF_F32>>(b, out, a, s);
+    } else if (mid_dt == WF_F16) lora_mid<WF_F16>(out_dt, qtype, b, out, a, s);
+    else if (mid_dt == WF_BF16) lora_mid<WF_BF16>(out_dt, qtype, b, out, a, s);
+    else lora_mid<WF_F32>(out_dt, qtype, b, out, a, s);
+    WF_LAUNCH_CHECK("wf_dequant_lora launch");
     return WF_OK;
 }

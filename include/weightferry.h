@@ -57,6 +57,15 @@ int wf_dequant(const void* src, int64_t src_bytes, int qtype, int mid_dt, int ou
 int wf_dequant_add(const void* src, int64_t src_bytes, int qtype, int mid_dt, int out_dt, const float* diff,
                    float scale, void* out, int64_t n_values, void* stream);
 
+/* The same add with the difference computed inside the kernel from the LoRA's factors: diff = up @ down in float32
+ * (up [n_out, rank] of dtype up_dt, down [rank, n_in] of dtype down_dt, both row-major on the device; float16 and
+ * bfloat16 are widened exactly), out [n_out, n_in]. src as in wf_dequant_add: NULL adds onto the values in out.
+ * rank 1..192; rows are whole blocks of qtype (a multiple of 8 values without src); out 16-byte aligned, down aligned
+ * to two of its values. */
+int wf_dequant_lora(const void* src, int64_t src_bytes, int qtype, int mid_dt, int out_dt, const void* up, int up_dt,
+                    const void* down, int down_dt, int64_t rank, float scale, void* out, int64_t n_out, int64_t n_in,
+                    void* stream);
+
 /* ---------------------------------------------------------------------------------------------- int8 W8A8 path
  * Per-row int8 quantisation of bf16 activations: replaces the Triton `_quant_row` with PRE_NONE
  * (enhancers/fused_kernels.py:137-174, launched at enhancers/fused_int8.py:172-176) and kitchen's

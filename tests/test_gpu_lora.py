@@ -68,6 +68,37 @@ def test_later_lora_onto_weight(native, out, n):
     assert ok, where
 
 
+# rows around the kernel's 32-row tiles, columns around its 256 (one block, a ragged last tile), odd and largest ranks
+@pytest.mark.parametrize("qtype,n_out,n_in,rank", [
+    (7, 1, 32, 1), (8, 33, 288, 7), (3, 31, 256, 8), (2, 64, 544, 33), (6, 40, 1024, 64), (12, 32, 256, 16),
+    (13, 65, 512, 2), (14, 33, 768, 24), (10, 7, 256, 192), (11, 96, 512, 5), (None, 33, 264, 12), (None, 3, 8, 192)])
+def test_lora_product_inside_the_kernel(native, qtype, n_out, n_in, rank):
+    # factors of small integers: every float32 sum of their products is exact, so the result is one set of bits
+    rng = np.random.default_rng(rank + n_in)
+    ups, downs = (rng.integers(-8, 9, s).astype(np.float32) for s in ((n_out, rank), (rank, n_in)))
+    diff = (ups.astype(np.float64) @ downs).astype(np.float32).ravel()
+    n = n_out * n_in
+    for mid, out in (PAIRS if qtype is not None else [(F16, o) for o in (F16, BF16, F32)]):
+        udt, ddt = TD[(mid + out) % 3], TD[out]
+        up, down = torch.from_numpy(ups).to("cuda", udt), torch.from_numpy(downs).to("cuda", ddt)
+        if qtype is not None:
+            raw = encode.random_blocks(qtype, n // encode.PER_BLOCK[qtype], seed=qtype, family="normal")
+            raw_dev, res = torch.from_numpy(raw).cuda(), torch.empty(n, dtype=TD[out], device="cuda")
+            blocks, expect = (raw_dev.data_ptr(), raw_dev.numel(), qtype, mid), lib.dequant_add(raw, qtype, mid, out, diff,
+                                                                                                0.0078125)
+        else:
+            w = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(TD[out])
+            res, blocks = w.cuda(), (None, 0, 0, 0)
+            expect = lib.dequant_add(None, 0, 0, out, diff, 0.0078125, base=_bits(w, out))
+        print(f"case qtype={qtype} {n_out}x{n_in} rank={rank} mid={mid} out={out}", flush=True)
+        rc = native.lib().wf_dequant_lora(*blocks, out, up.data_ptr(), (mid + out) % 3, down.data_ptr(), out, rank,
+                                          0.0078125, res.data_ptr(), n_out, n_in, native.stream_of(res.device))
+        assert rc == 0, native.last_error()
+        torch.cuda.synchronize()
+        ok, where = _same(_bits(res, out), expect, out)
+        assert ok, (mid, out, where)
+
+
 class LoRAAdapter:
     def __init__(self, weights):
         self.weights = weights
