@@ -48,6 +48,43 @@ struct Residual {
     int rows_per_group;
 };
 
+// The residual form's last step on the plain form's bf16 outputs (already in LDS rows): whole 16-byte runs of residual
+// and gate, the residual loaded before the tile is written to LDS. With element loads and stores of 2 bytes in the MFMA
+// layout the epilogue waited on 16 loads a tile row in turn: 5152 x 2048 x 8192 took 139 us against 102 now (98 without
+// the residual), 4096 x 5120 x 5120 156 against 103 (95), 500 x 2048 x 8192 57.6 against 40.2 (35.8).
+struct AddResidual {
+    typedef uint4 Fetched;
+    const Residual r;
+    const int N;
+    const bool vec_ok;
+    __device__ __forceinline__ AddResidual(const Residual& res, int n)
+        : r(res), N(n), vec_ok(((reinterpret_cast<uintptr_t>(res.gate) | reinterpret_cast<uintptr_t>(res.resid)) & 15) == 0) {}
+    static __device__ __forceinline__ float lo(uint32_t u) { return __uint_as_float(u << 16); }
+    static __device__ __forceinline__ float hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
+    __device__ __forceinline__ uint4 prefetch(int m, int n) const {
+        return *reinterpret_cast<const uint4*>(r.resid + (int64_t)m * N + n);
+    }
+    __device__ __forceinline__ uint4 run(uint4 v, const uint4& x, int m, int n) const {
+        const uint4 g = *reinterpret_cast<const uint4*>(r.gate + (int64_t)(m / r.rows_per_group) * N + n);
+        const uint32_t tv[4] = {v.x, v.y, v.z, v.w}, xv[4] = {x.x, x.y, x.z, x.w}, gv[4] = {g.x, g.y, g.z, g.w};
+        uint32_t o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            o[e] = pack_bf16(lo(xv[e]) + lo(gv[e]) * lo(tv[e]), hi(xv[e]) + hi(gv[e]) * hi(tv[e]));
+        return make_uint4(o[0], o[1], o[2], o[3]);
+    }
+    __device__ __forceinline__ uint16_t one(uint16_t t, int m, int n) const {
+        const float g = lo(r.gate[(int64_t)(m / r.rows_per_group) * N + n]), x = lo(r.resid[(int64_t)m * N + n]);
+        return __builtin_bit_cast(uint16_t, (__bf16)(x + g * lo(t)));
+    }
+};
+
+template <bool RESID>
+__device__ __forceinline__ auto last_step(const Residual& res, int N) {
+    if constexpr (RESID) return AddResidual(res, N);
+    else return StoreAsIs{};
+}
+
 // The per-row activation scales of a wave's R = 32 WM output rows from row mw: lane l loads xs[mw + l] (and
 // xs[mw + 64 + l] for R = 128), one load each; row(ro) gives any lane the scale of row mw + ro by a lane permute
 // (ds_bpermute). A global load per output element instead left each tile's epilogue waiting on 16-32 loads in
@@ -339,93 +376,60 @@ __global__ __launch_bounds__(64 * VM * VN) void gemm_i8_dl(const int8_t* __restr
     if (kt + 2 < nk) step(kt + 2, st2, st3, st1);
 
     // epilogue: (float(acc) * xs[m]) * ws[n] (+ bias[n]), rounded once to OUT
-    if constexpr (!RESID) {
-        // Through LDS: each wave writes its WM*32 x WN*32 tile, rounded, into its own LDS region (row-major,
-        // WN*32 values a row), then stores whole 16-byte runs of output rows. The ring is idle by now: every
-        // wave's last loads have landed (s_waitcnt) and every wave is past its last fragment reads (barrier).
-        constexpr int TR = WM * 32, TC = WN * 32;          // this wave's rows and columns
-        constexpr int PER_BUF = SLOTS * 16 / (TR * TC * 2); // wave regions per ring buffer
-        static_assert(PER_BUF >= 1 && NW <= PER_BUF * 4, "the output tiles fit in the ring");
-        __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0)
-        wave_barrier_sync();
-        const int wb = wave / PER_BUF;
-        i32x4* buf = wb == 0 ? st0 : wb == 1 ? st1 : wb == 2 ? st2 : st3;
-        uint16_t* ot = reinterpret_cast<uint16_t*>(buf) + (wave % PER_BUF) * TR * TC;
-#pragma unroll
-        for (int j = 0; j < WN; j++) {
-#pragma unroll
-            for (int i = 0; i < WM; i++) {
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int r0 = i * 32 + 8 * q + 4 * lk;    // rows r0 .. r0 + 3 of this wave's tile
-                    float xm[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) xm[e] = rs.row(r0 + e);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        float t = ((float)acc[i][j][4 * q + e] * xm[e]) * wsn[j];
-                        if (BIAS) t = t + bn[j];
-                        ot[(r0 + e) * TC + j * 32 + lr] = OUT == WF_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)t)
-                                                                         : __builtin_bit_cast(uint16_t, (_Float16)t);
-                    }
-                }
-            }
-        }
-        // the wave reads back only its own region: its LDS writes and reads execute in order
-        const uint4* ov = reinterpret_cast<const uint4*>(ot);
-        constexpr int RUNS = TC / 8;                       // 16-byte runs per row
-        uint16_t* Y = static_cast<uint16_t*>(out);
-        if ((N & 7) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0) {   // whole aligned 16-byte runs
-#pragma unroll
-            for (int it = 0; it < TR * RUNS / 64; it++) {
-                const int q = it * 64 + lane, r = q / RUNS, c = q % RUNS;
-                const int m = mw + r, n = nw + 8 * c;
-                const uint4 v = ov[q];
-                if (m < M && n < N) *reinterpret_cast<uint4*>(Y + (int64_t)m * N + n) = v;   // N % 8: whole runs
-            }
-        } else {
-            for (int it = 0; it < TR * RUNS / 64; it++) {
-                const int q = it * 64 + lane, r = q / RUNS, c = q % RUNS;
-                const int m = mw + r;
-                if (m >= M) continue;
-                const uint16_t* row = ot + r * TC + 8 * c;
-                for (int e = 0; e < 8; e++) {
-                    const int n = nw + 8 * c + e;
-                    if (n < N) Y[(int64_t)m * N + n] = row[e];
-                }
-            }
-        }
-        return;
-    }
-    // the residual form: element stores, once the ring's last loads (stages past K among them) have landed -- no
-    // copy into this workgroup's LDS may outlive it
-    // (every lane reaches each row permute: a lane that skipped it would hand a zero to the lanes reading its row)
+    // Through LDS: each wave writes its WM*32 x WN*32 tile, rounded, into its own LDS region (row-major,
+    // WN*32 values a row), then stores whole 16-byte runs of output rows. The ring is idle by now: every
+    // wave's last loads have landed (s_waitcnt) and every wave is past its last fragment reads (barrier).
+    constexpr int TR = WM * 32, TC = WN * 32;          // this wave's rows and columns
+    constexpr int PER_BUF = SLOTS * 16 / (TR * TC * 2); // wave regions per ring buffer
+    static_assert(PER_BUF >= 1 && NW <= PER_BUF * 4, "the output tiles fit in the ring");
     __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0)
+    wave_barrier_sync();
+    const int wb = wave / PER_BUF;
+    i32x4* buf = wb == 0 ? st0 : wb == 1 ? st1 : wb == 2 ? st2 : st3;
+    uint16_t* ot = reinterpret_cast<uint16_t*>(buf) + (wave % PER_BUF) * TR * TC;
 #pragma unroll
     for (int j = 0; j < WN; j++) {
-        const int n = nw + j * 32 + lr;
-        const bool in_n = n < N;
 #pragma unroll
         for (int i = 0; i < WM; i++) {
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int ro = i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3);
-                const int m = mw + ro;
-                const float xm = rs.row(ro);
-                if (!in_n || m >= M) continue;
-                float t = ((float)acc[i][j][e] * xm) * wsn[j];
-                if (BIAS) t = t + bn[j];
-                const int64_t o = (int64_t)m * N + n;
-                if constexpr (RESID) {
-                    const float g = __uint_as_float((uint32_t)res.gate[(int64_t)(m / res.rows_per_group) * N + n] << 16);
-                    const float r = __uint_as_float((uint32_t)res.resid[o] << 16);
-                    t = r + g * (float)(__bf16)t;
+            for (int q = 0; q < 4; q++) {
+                const int r0 = i * 32 + 8 * q + 4 * lk;    // rows r0 .. r0 + 3 of this wave's tile
+                float xm[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) xm[e] = rs.row(r0 + e);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float t = ((float)acc[i][j][4 * q + e] * xm[e]) * wsn[j];
+                    if (BIAS) t = t + bn[j];
+                    ot[(r0 + e) * TC + j * 32 + lr] = OUT == WF_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)t)
+                                                                     : __builtin_bit_cast(uint16_t, (_Float16)t);
                 }
-                if constexpr (OUT == WF_BF16) {
-                    static_cast<__bf16*>(out)[o] = (__bf16)t;
-                } else {
-                    static_cast<_Float16*>(out)[o] = (_Float16)t;
-                }
+            }
+        }
+    }
+    // the wave reads back only its own region: its LDS writes and reads execute in order
+    const uint4* ov = reinterpret_cast<const uint4*>(ot);
+    constexpr int RUNS = TC / 8;                       // 16-byte runs per row
+    uint16_t* Y = static_cast<uint16_t*>(out);
+    const auto fin = last_step<RESID>(res, N);
+    if ((N & 7) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0 && fin.vec_ok) {   // whole aligned 16-byte runs
+#pragma unroll
+        for (int it = 0; it < TR * RUNS / 64; it++) {
+            const int q = it * 64 + lane, r = q / RUNS, c = q % RUNS;
+            const int m = mw + r, n = nw + 8 * c;
+            const uint4 v = ov[q];
+            if (m < M && n < N)                            // N % 8: whole runs
+                *reinterpret_cast<uint4*>(Y + (int64_t)m * N + n) = fin.run(v, fin.prefetch(m, n), m, n);
+        }
+    } else {
+        for (int it = 0; it < TR * RUNS / 64; it++) {
+            const int q = it * 64 + lane, r = q / RUNS, c = q % RUNS;
+            const int m = mw + r;
+            if (m >= M) continue;
+            const uint16_t* row = ot + r * TC + 8 * c;
+            for (int e = 0; e < 8; e++) {
+                const int n = nw + 8 * c + e;
+                if (n < N) Y[(int64_t)m * N + n] = fin.one(row[e], m, n);
             }
         }
     }
@@ -434,8 +438,7 @@ __global__ __launch_bounds__(64 * VM * VN) void gemm_i8_dl(const int8_t* __restr
 // K % 128 == 0, the 256-row tilings: whole 128-byte lines through two stage buffers (wl_ring.h), whose barrier sits
 // before the last K step's MFMAs and whose loads leave right after it (16384 x 13824 x 5120: 1049 against 1137 us
 // for the 64-byte ring, 4096 x 5120 x 5120: 100.1 against 105.4 us). The 128 x 160 tiling keeps the 4-stage ring of
-// 128-byte stages (1024 x 5120 x 5120: 35.5 against 38.3 us on two buffers). Epilogue as above; the residual form
-// stores single elements.
+// 128-byte stages (1024 x 5120 x 5120: 35.5 against 38.3 us on two buffers). Epilogue as above.
 template <typename S, int OUT, bool BIAS, bool RESID>
 __global__ __launch_bounds__(S::NT) void gemm_i8_wl(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
                                                     const float* __restrict__ xs, const float* __restrict__ ws,
@@ -474,37 +477,15 @@ __global__ __launch_bounds__(S::NT) void gemm_i8_wl(const int8_t* __restrict__ A
         bn[j] = BIAS && n < N ? to_f32_out(bias, n, OUT) : 0.0f;
     }
     const RowScales<WM> rs(xs, mw, M, lane);
-    if constexpr (!RESID) {
-        wl_store_tile<WM, WN>(wl_out_region<S>(sb0, sb1, wave), static_cast<uint16_t*>(out), M, N, mw, nw, lane,
-                              [&](int i, int j, int e) {
-                                  const float xm = rs.row(i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3));
-                                  float t = ((float)acc[i][j][e] * xm) * wsn[j];
-                                  if (BIAS) t = t + bn[j];
-                                  return OUT == WF_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)t)
-                                                        : __builtin_bit_cast(uint16_t, (_Float16)t);
-                              });
-    } else {
-        // (every lane reaches each row permute: a lane that skipped it would hand a zero to the lanes reading its row)
-#pragma unroll
-        for (int j = 0; j < WN; j++) {
-            const int n = nw + j * 32 + lr;
-#pragma unroll
-            for (int i = 0; i < WM; i++) {
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int ro = i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3);
-                    const int m = mw + ro;
-                    const float xm = rs.row(ro);
-                    if (n >= N || m >= M) continue;
-                    const float t = ((float)acc[i][j][e] * xm) * wsn[j];
-                    const int64_t o = (int64_t)m * N + n;
-                    const float g = __uint_as_float((uint32_t)res.gate[(int64_t)(m / res.rows_per_group) * N + n] << 16);
-                    const float r = __uint_as_float((uint32_t)res.resid[o] << 16);
-                    static_cast<__bf16*>(out)[o] = (__bf16)(r + g * (float)(__bf16)t);
-                }
-            }
-        }
-    }
+    wl_store_tile<WM, WN>(
+        wl_out_region<S>(sb0, sb1, wave), static_cast<uint16_t*>(out), M, N, mw, nw, lane,
+        [&](int i, int j, int e) {
+            const float xm = rs.row(i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3));
+            float t = ((float)acc[i][j][e] * xm) * wsn[j];
+            if (BIAS) t = t + bn[j];
+            return OUT == WF_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)t) : __builtin_bit_cast(uint16_t, (_Float16)t);
+        },
+        last_step<RESID>(res, N));
 }
 
 template <int VM, int VN, int WM, int WN, int OUT>

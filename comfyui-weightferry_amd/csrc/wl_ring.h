@@ -118,42 +118,61 @@ __device__ __forceinline__ uint16_t* wl_out_region(wl_frag* sb0, wl_frag* sb1, i
     return reinterpret_cast<uint16_t*>(wave / PER_BUF == 0 ? sb0 : sb1) + (wave % PER_BUF) * 32 * S::WN * 32;
 }
 
+// What wl_store_tile does to a finished run of 8 outputs before it is stored; this one leaves it as it is. prefetch(m,
+// n) loads what the run at row m, column n needs (in range), run(v, f, m, n) combines it; one(v, m, n) does the same
+// to a single value.
+struct StoreAsIs {
+    struct Fetched {};
+    static constexpr bool vec_ok = true;
+    __device__ __forceinline__ Fetched prefetch(int, int) const { return {}; }
+    __device__ __forceinline__ uint4 run(uint4 v, const Fetched&, int, int) const { return v; }
+    __device__ __forceinline__ uint16_t one(uint16_t v, int, int) const { return v; }
+};
+
 // Stores the wave's WM * 32 x WN * 32 output tile at rows mw.., columns nw.. of Y [M, N] (16-bit values), 32 rows at
 // a time through its LDS region ot: bits(i, j, e) gives the output bits of accumulator element e of MFMA tile (i, j)
-// (row mw + 32 i + 8 (e / 4) + 4 (lane / 32) + e % 4, column nw + 32 j + lane % 32). Whole 16-byte row runs go out
-// when N % 8 == 0 and Y is 16-byte aligned, single values otherwise. The wave reads back only its own region, and its
-// LDS writes and reads execute in order.
-template <int WM, int WN, typename Bits>
+// (row mw + 32 i + 8 (e / 4) + 4 (lane / 32) + e % 4, column nw + 32 j + lane % 32), fin's run() or one() the value
+// stored. Whole 16-byte row runs go out when N % 8 == 0 and Y is 16-byte aligned, single values otherwise. The wave
+// reads back only its own region, and its LDS writes and reads execute in order.
+template <int WM, int WN, typename Bits, typename Fin = StoreAsIs>
 __device__ __forceinline__ void wl_store_tile(uint16_t* ot, uint16_t* Y, int M, int N, int mw, int nw, int lane,
-                                              Bits&& bits) {
-    constexpr int TC = WN * 32, RUNS = TC / 8;
+                                              Bits&& bits, const Fin& fin = Fin{}) {
+    constexpr int TC = WN * 32, RUNS = TC / 8, NIT = 32 * RUNS / 64;
     const int lr = lane & 31, lk = lane >> 5;
     const uint4* ov = reinterpret_cast<const uint4*>(ot);
-    const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
+    const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0 && fin.vec_ok;
 #pragma unroll
     for (int i = 0; i < WM; i++) {
         const int mi = mw + i * 32;
+        typename Fin::Fetched f[NIT];
+        if (vec) {
+#pragma unroll
+            for (int it = 0; it < NIT; it++) {
+                const int q = it * 64 + lane;
+                f[it] = fin.prefetch(min(mi + q / RUNS, M - 1), min(nw + 8 * (q % RUNS), N - 8));
+            }
+        }
 #pragma unroll
         for (int e = 0; e < 16; e++)
 #pragma unroll
             for (int j = 0; j < WN; j++) ot[(8 * (e >> 2) + 4 * lk + (e & 3)) * TC + j * 32 + lr] = bits(i, j, e);
         if (vec) {
 #pragma unroll
-            for (int it = 0; it < 32 * RUNS / 64; it++) {
+            for (int it = 0; it < NIT; it++) {
                 const int q = it * 64 + lane, r = q / RUNS, c = q % RUNS;
                 const int m = mi + r, n = nw + 8 * c;
                 const uint4 v = ov[q];
-                if (m < M && n < N) *reinterpret_cast<uint4*>(Y + (int64_t)m * N + n) = v;
+                if (m < M && n < N) *reinterpret_cast<uint4*>(Y + (int64_t)m * N + n) = fin.run(v, f[it], m, n);
             }
         } else {
-            for (int it = 0; it < 32 * RUNS / 64; it++) {
+            for (int it = 0; it < NIT; it++) {
                 const int q = it * 64 + lane, r = q / RUNS, c = q % RUNS;
                 const int m = mi + r;
                 if (m >= M) continue;
                 const uint16_t* row = ot + r * TC + 8 * c;
                 for (int e = 0; e < 8; e++) {
                     const int n = nw + 8 * c + e;
-                    if (n < N) Y[(int64_t)m * N + n] = row[e];
+                    if (n < N) Y[(int64_t)m * N + n] = fin.one(row[e], m, n);
                 }
             }
         }

@@ -369,3 +369,28 @@ def test_pending_layernorm_at_a_width_that_is_not_a_power_of_two_is_materialised
     rq, rs = lib.quant_rows(_bits(real.reshape(-1, K)), 1)
     expect = lib.linear_i8(rq, w_q.numpy(), rs, ws.numpy(), out_dt=lib.BF16)
     assert np.array_equal(_bits(y.reshape(-1, 256)), expect)
+
+
+@pytest.mark.parametrize("M,N,K,off", [(64, 8, 128, 0), (6, 4, 128, 0), (258, 264, 256, 0), (258, 264, 256, 1),
+                                       (130, 24, 192, 1), (2, 1, 64, 0)])
+def test_residual_runs_and_single_values(native, M, N, K, off):
+    # whole 16-byte runs of residual and gate where every address allows it (N % 8 == 0, off 0), single values
+    # elsewhere (off: the residual and the gate start 2 bytes into their buffers); M ends inside a tile-row
+    g = torch.Generator().manual_seed(N + K + off)
+    xq, wq = _rand_i8(g, (M, K)), _rand_i8(g, (N, K))
+    xs, ws = torch.rand(M, generator=g) * 0.05 + 1e-3, torch.rand(N, generator=g) * 0.002 + 1e-5
+    gate, resid = torch.randn((2, N), generator=g).to(torch.bfloat16), torch.randn((M, N), generator=g).to(torch.bfloat16)
+    t = (((xq.double() @ wq.double().T).float() * xs[:, None]) * ws[None, :]).to(torch.bfloat16)
+    ref = torch.addcmul(resid, gate.repeat_interleave(M // 2, 0), t)
+
+    def shifted(v):
+        buf = torch.zeros(v.numel() + 8, dtype=v.dtype, device="cuda")
+        buf[off:off + v.numel()] = v.reshape(-1).cuda()
+        return buf[off:]
+    d = [v.cuda() for v in (xq, wq, xs, ws)]
+    gd, rd, y = shifted(gate), shifted(resid), torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    rc = native.lib().wf_linear_i8_residual(*[v.data_ptr() for v in d], gd.data_ptr(), rd.data_ptr(), y.data_ptr(), M, N, K,
+                                            M // 2, native.stream_of(y.device))
+    assert rc == 0, native.last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(y.cpu().view(torch.int16), ref.view(torch.int16))
