@@ -39,7 +39,7 @@ __global__ __launch_bounds__(S::NT) void gemm_bf16(const uint16_t* __restrict__ 
         for (int j = 0; j < WN; j++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
-    wl_mainloop<S>(ra, rb, KB, (int)(KB / 128), wave, lane, sb0, sb1, acc,
+    wl_mainloop<S>(ra, rb, KB, 0, (int)(KB / 128), wave, lane, sb0, sb1, acc,
                    [](const f32x16v& c, const wl_frag& a, const wl_frag& b) {
                        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8v, a),
                                                                       __builtin_bit_cast(bf16x8v, b), c, 0, 0, 0);

@@ -461,7 +461,7 @@ __global__ __launch_bounds__(S::NT) void gemm_i8_wl(const int8_t* __restrict__ A
         for (int j = 0; j < WN; j++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0;
-    wl_mainloop<S>(ra, rb, (uint32_t)K, K / 128, wave, lane, sb0, sb1, acc,
+    wl_mainloop<S>(ra, rb, (uint32_t)K, 0, K / 128, wave, lane, sb0, sb1, acc,
                    [](const i32x16& c, const wl_frag& a, const wl_frag& b) {
                        return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
                    });
