@@ -5,11 +5,13 @@
 // at K offset 16 * (l / 32) of the 32-wide K step. Result layout: lane l, register i holds row 8 (i / 4) +
 // 4 (l / 32) + i % 4, column l % 32 of the 32x32 tile.
 //
-// Two kernels:
-//  * gemm_i8_dl (K % 64 == 0, the workload): 256 x 320, 256 x 256, 256 x 128 or 128 x 160 tiles (chosen per
-//    shape, see launch_dl), operands streamed global -> LDS by the load unit (no register staging) through a
-//    4-stage ring of 64-byte K stages (128-byte for 128 x 160 tiles), and an epilogue that stages the rounded
-//    tile in LDS and stores whole 16-byte runs of output rows.
+// Kernels:
+//  * gemm_i8_wl (K % 128 == 0): tiles of 32 x 128 to 256 x 320 over two LDS stage buffers (wl_ring.h), and
+//    gemm_i8_part + gemm_i8_sum, the same loop over slices of K where the tiles alone leave CUs idle (i8_plan).
+//  * gemm_i8_dl (K % 64 == 0; of K % 128 == 0 the 128 x 160 tiles only): 256 x 320, 256 x 256, 256 x 128 or
+//    128 x 160 tiles (chosen per shape, see launch_dl), operands streamed global -> LDS by the load unit (no
+//    register staging) through a 4-stage ring of 64-byte K stages (128-byte for 128 x 160 tiles), and an epilogue
+//    that stages the rounded tile in LDS and stores whole 16-byte runs of output rows.
 //  * gemm_i8 (K % 16 == 0 otherwise): 2 x 2 waves, predicated loads staged through registers into a
 //    double-buffered LDS tile of 128-byte K stages. Rows are 8 chunks of 16 bytes; chunk c of row r sits at slot
 //    c ^ (((r >> 1) ^ ((r & 1) << 2)) & 7), conflict-free for stage writes and fragment reads.
@@ -435,6 +437,32 @@ __global__ __launch_bounds__(64 * VM * VN) void gemm_i8_dl(const int8_t* __restr
     }
 }
 
+// Scales, bias, rounding, last step and stores of a wave's WM x WN MFMA tiles at rows mw.., columns nw.., through its
+// LDS region ot (32 rows of WN * 32 values).
+template <int WM, int WN, int OUT, bool BIAS, bool RESID>
+__device__ __forceinline__ void i8_outputs(const i32x16 (&acc)[WM][WN], uint16_t* ot, const float* __restrict__ xs,
+                                           const float* __restrict__ ws, const void* __restrict__ bias, void* out, int M,
+                                           int N, int mw, int nw, int lane, const Residual& res) {
+    const int lr = lane & 31, lk = lane >> 5;
+    float wsn[WN], bn[WN];
+#pragma unroll
+    for (int j = 0; j < WN; j++) {
+        const int n = nw + j * 32 + lr;
+        wsn[j] = n < N ? ws[n] : 0.0f;
+        bn[j] = BIAS && n < N ? to_f32_out(bias, n, OUT) : 0.0f;
+    }
+    const RowScales<WM> rs(xs, mw, M, lane);
+    wl_store_tile<WM, WN>(
+        ot, static_cast<uint16_t*>(out), M, N, mw, nw, lane,
+        [&](int i, int j, int e) {
+            const float xm = rs.row(i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3));
+            float t = ((float)acc[i][j][e] * xm) * wsn[j];
+            if (BIAS) t = t + bn[j];
+            return OUT == WF_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)t) : __builtin_bit_cast(uint16_t, (_Float16)t);
+        },
+        last_step<RESID>(res, N));
+}
+
 // K % 128 == 0, the 256-row tilings: whole 128-byte lines through two stage buffers (wl_ring.h), whose barrier sits
 // before the last K step's MFMAs and whose loads leave right after it (16384 x 13824 x 5120: 1049 against 1137 us
 // for the 64-byte ring, 4096 x 5120 x 5120: 100.1 against 105.4 us). The 128 x 160 tiling keeps the 4-stage ring of
@@ -466,26 +494,84 @@ __global__ __launch_bounds__(S::NT) void gemm_i8_wl(const int8_t* __restrict__ A
                        return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
                    });
     // (the scales load after the main loop here: held through it, the 256-row tilings' accumulators spill)
-    const int wm = wave / S::VN, wn = wave % S::VN;
-    const int mw = m0 + wm * WM * 32, nw = n0 + wn * WN * 32;
-    const int lr = lane & 31, lk = lane >> 5;
-    float wsn[WN], bn[WN];
+    const int mw = m0 + wave / S::VN * WM * 32, nw = n0 + wave % S::VN * WN * 32;
+    i8_outputs<WM, WN, OUT, BIAS, RESID>(acc, wl_out_region<S>(sb0, sb1, wave), xs, ws, bias, out, M, N, mw, nw, lane, res);
+}
+
+// ------------------------------------------------------------------------------------------ K in slices
+// Products whose tiles leave CUs idle: blockIdx.y is a slice of `per` 128-byte K stages, whose int32 sums go to part in
+// the MFMA's own layout (16 bytes a lane, 1 KiB a wave store); gemm_i8_sum adds the slices, an exact sum in any order,
+// and runs the epilogue, one wave a 32 x 32 tile. Up to 512 rows a tile's chain of stage after stage set the time: 30 us
+// for 40 stages of 128 x 160 tiles on 32-128 of the 256 CUs.
+template <typename S>
+__global__ __launch_bounds__(S::NT) void gemm_i8_part(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
+                                                      i32x4* __restrict__ part, int M, int N, int K, int per) {
+    constexpr int WM = S::WM, WN = S::WN;
+    __shared__ wl_frag sb0[S::SLOTS], sb1[S::SLOTS];
+    const int ntm = (M + S::BM - 1) / S::BM, ntn = (N + S::BN - 1) / S::BN;
+    int tm, tn;
+    tile_order(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
+    const int m0 = __builtin_amdgcn_readfirstlane(tm * S::BM), n0 = __builtin_amdgcn_readfirstlane(tn * S::BN);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const __amdgpu_buffer_rsrc_t ra = tile_rsrc(A + (int64_t)m0 * K, (int64_t)(M - m0) * K);
+    const __amdgpu_buffer_rsrc_t rb = tile_rsrc(B + (int64_t)n0 * K, (int64_t)(N - n0) * K);
+    i32x16 acc[WM][WN];
 #pragma unroll
-    for (int j = 0; j < WN; j++) {
-        const int n = nw + j * 32 + lr;
-        wsn[j] = n < N ? ws[n] : 0.0f;
-        bn[j] = BIAS && n < N ? to_f32_out(bias, n, OUT) : 0.0f;
+    for (int i = 0; i < WM; i++)
+#pragma unroll
+        for (int j = 0; j < WN; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0;
+    const int s0 = (int)blockIdx.y * per;
+    wl_mainloop<S>(ra, rb, (uint32_t)K, s0, min(per, K / 128 - s0), wave, lane, sb0, sb1, acc,
+                   [](const i32x16& c, const wl_frag& a, const wl_frag& b) {
+                       return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+                   });
+    const int64_t tile = (int64_t)blockIdx.y * (ntm * ntn) + tm * ntn + tn;
+    i32x4* p = part + (tile * S::NW + wave) * (WM * WN * 256) + lane;
+#pragma unroll
+    for (int i = 0; i < WM; i++)
+#pragma unroll
+        for (int j = 0; j < WN; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                i32x4 v;
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * q + e];
+                p[((i * WN + j) * 4 + q) * 64] = v;
+            }
+}
+
+template <typename S, int OUT, bool BIAS, bool RESID>
+__global__ __launch_bounds__(256) void gemm_i8_sum(const i32x4* __restrict__ part, const float* __restrict__ xs,
+                                                   const float* __restrict__ ws, const void* __restrict__ bias,
+                                                   void* __restrict__ out, int M, int N, int tiles, int slices,
+                                                   Residual res) {
+    constexpr int WM = S::WM, WN = S::WN, PER_TILE = S::NW * WM * WN;
+    __shared__ __attribute__((aligned(16))) uint16_t rows[4][32 * 32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t f = (int64_t)blockIdx.x * 4 + wave, all = (int64_t)tiles * PER_TILE;
+    if (f >= all) return;
+    const int ntn = (N + S::BN - 1) / S::BN;
+    const int tile = (int)(f / PER_TILE), in = (int)(f % PER_TILE);
+    const int w = in / (WM * WN), i = in % (WM * WN) / WN, j = in % WN;
+    const int mw = tile / ntn * S::BM + (w / S::VN * WM + i) * 32, nw = tile % ntn * S::BN + (w % S::VN * WN + j) * 32;
+    if (mw >= M || nw >= N) return;
+    const i32x4* p = part + f * 256 + lane;
+    i32x4 a[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) a[q] = p[q * 64];
+#pragma unroll 3
+    for (int s = 1; s < slices; s++) {
+        const i32x4* ps = p + (int64_t)s * all * 256;
+#pragma unroll
+        for (int q = 0; q < 4; q++) a[q] += ps[q * 64];
     }
-    const RowScales<WM> rs(xs, mw, M, lane);
-    wl_store_tile<WM, WN>(
-        wl_out_region<S>(sb0, sb1, wave), static_cast<uint16_t*>(out), M, N, mw, nw, lane,
-        [&](int i, int j, int e) {
-            const float xm = rs.row(i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3));
-            float t = ((float)acc[i][j][e] * xm) * wsn[j];
-            if (BIAS) t = t + bn[j];
-            return OUT == WF_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)t) : __builtin_bit_cast(uint16_t, (_Float16)t);
-        },
-        last_step<RESID>(res, N));
+    i32x16 acc[1][1];
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[0][0][e] = a[e >> 2][e & 3];
+    i8_outputs<1, 1, OUT, BIAS, RESID>(acc, rows[wave], xs, ws, bias, out, M, N, mw, nw, lane, res);
 }
 
 template <int VM, int VN, int WM, int WN, int OUT>
@@ -540,10 +626,108 @@ static void launch_dl(const int8_t* A, const int8_t* B, const float* xs, const f
     else launch_dl_shape<4, 2, 2, 5, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
 }
 
+// ---- K % 128 == 0 and less than one round of 256 x 320 tiles: tiling and slices by a modelled time
+struct I8Form {
+    int bm, bn;          // tile
+    int stage, turn;     // ns of a 128-byte stage: alone on a CU; its share of the CU when a CU has several workgroups
+};
+// Times fitted on MI355X to 1,900 measurements (rows 4-5152, 1024 <= N, K <= 13824, weights out of the last-level
+// cache); over them the choice is 1.40 times as fast as the 256-row and 128 x 160 tilings alone and within 3 % of the
+// best form measured, and one shape in 130 is over 1 % slower than before (1536 x 2048 x 8192, 4 %). Against the tilings
+// alone (us): 5120 x 5120 at 16 / 64 / 128 / 256 / 512 rows 13.3 / 15.2 / 17.5 / 23.3 / 32.7 against 27.9 / 29.6 / 33.7
+// / 33.0 / 32.7; 5120 x 13824 at 16 / 256 / 768 rows 23.8 / 38.9 / 70.5 against 66.4 / 76.2 / 78.2; 2048 x 8192 at 256
+// rows 17.4 against 44.7; 1024 x 1024 at 64 rows 4.7 against 9.0.
+constexpr I8Form kI8Forms[] = {{32, 128, 705, 394},    {64, 128, 806, 460},    {128, 128, 900, 562},
+                               {256, 192, 1334, 1276}, {256, 256, 1481, 1486}, {256, 320, 1667, 1608}};
+// ns of a 256 x 256 tile's epilogue; of the sums' launch; bytes per ns of the slices' way through memory and of a
+// weight's, which also costs kI8Start
+constexpr int64_t kI8Epilogue = 2992, kI8Sum = 4523, kI8SumBytes = 6804, kI8Stream = 4854, kI8Start = 3000;
+constexpr int kI8Ring = 6;                      // gemm_i8_dl's 128 x 160 tiles, 4-stage ring
+constexpr int kI8MinStages = 3, kI8MaxSlices = 16;
+
+struct I8Plan {
+    int form, slices, per;
+    int64_t part_bytes;
+};
+
+static int64_t tiles_of(int64_t M, int64_t N, int bm, int bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); }
+
+constexpr int64_t kI8MaxPart = 128LL << 20;
+
+// modelled ns of a form over `tiles` tiles in `slices` slices of `per` stages, and of the 128 x 160 ring
+static int64_t i8_time(const I8Form& F, int64_t tiles, int64_t slices, int64_t per, int64_t weight_bytes) {
+    const int64_t turns = (tiles * slices + 255) / 256, area = (int64_t)F.bm * F.bn;
+    const int64_t loop = per * (turns == 1 ? F.stage : turns * F.turn) + turns * area * kI8Epilogue / 65536;
+    const int64_t sums = slices > 1 ? kI8Sum + tiles * slices * area * 8 / kI8SumBytes : 0;
+    return std::max(loop, weight_bytes / kI8Stream + kI8Start) + sums;
+}
+static int64_t i8_ring_time(int64_t tiles, int64_t nk) { return 4000 + (tiles + 255) / 256 * nk * 640; }
+
+static bool i8_modelled(int64_t M, int64_t N, int64_t K) { return K % 128 == 0 && tiles_of(M, N, 256, 320) < 256; }
+
+static I8Plan i8_plan(int64_t M, int64_t N, int64_t K, int64_t max_part) {
+    const int64_t nk = K / 128;
+    I8Plan best{kI8Ring, 1, (int)nk, 0};
+    int64_t t = INT64_MAX;
+    for (int f = 0; f < 6; f++) {
+        const I8Form& F = kI8Forms[f];
+        const int64_t tiles = tiles_of(M, N, F.bm, F.bn);
+        int64_t last = 0;
+        for (int s = 1; s <= kI8MaxSlices; s++) {
+            const int64_t per = (nk + s - 1) / s, slices = (nk + per - 1) / per;
+            if (s > 1 && (per < kI8MinStages || slices == last || tiles * slices > 1024)) continue;
+            last = slices;
+            const int64_t part = slices > 1 ? tiles * slices * F.bm * F.bn * 4 : 0;
+            if (part > std::min(max_part, kI8MaxPart)) continue;
+            const int64_t v = i8_time(F, tiles, slices, per, N * K);
+            if (v < t) { t = v; best = {f, (int)slices, (int)per, part}; }
+        }
+    }
+    if (i8_ring_time(tiles_of(M, N, 128, 160), nk) < t) best = {kI8Ring, 1, (int)nk, 0};
+    return best;
+}
+
+template <int VM, int VN, int WM, int WN, int OUT>
+static void launch_i8_form(const I8Plan& p, const int8_t* A, const int8_t* B, const float* xs, const float* ws,
+                           const void* bias, void* out, int M, int N, int K, Residual r, bool resid, void* part,
+                           hipStream_t s) {
+    using S = WlShape<VM, VN, WM, WN>;
+    if (p.slices == 1) {
+        launch_wl_shape<VM, VN, WM, WN, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
+        return;
+    }
+    const int tiles = (int)tiles_of(M, N, S::BM, S::BN);
+    const dim3 sum((unsigned)(((int64_t)tiles * S::NW * WM * WN + 3) / 4));
+    i32x4* P = static_cast<i32x4*>(part);
+    gemm_i8_part<S><<<dim3(tiles, p.slices), S::NT, 0, s>>>(A, B, P, M, N, K, p.per);
+    if (resid) gemm_i8_sum<S, OUT, false, true><<<sum, 256, 0, s>>>(P, xs, ws, nullptr, out, M, N, tiles, p.slices, r);
+    else if (bias) gemm_i8_sum<S, OUT, true, false><<<sum, 256, 0, s>>>(P, xs, ws, bias, out, M, N, tiles, p.slices, r);
+    else gemm_i8_sum<S, OUT, false, false><<<sum, 256, 0, s>>>(P, xs, ws, bias, out, M, N, tiles, p.slices, r);
+}
+
+template <int OUT>
+static void launch_i8_plan(const I8Plan& p, const int8_t* A, const int8_t* B, const float* xs, const float* ws,
+                           const void* bias, void* out, int M, int N, int K, Residual r, bool resid, void* part,
+                           hipStream_t s) {
+    switch (p.form) {
+    case 0: launch_i8_form<1, 4, 1, 1, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
+    case 1: launch_i8_form<1, 4, 2, 1, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
+    case 2: launch_i8_form<2, 4, 2, 1, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
+    case 3: launch_i8_form<4, 2, 2, 3, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
+    case 4: launch_i8_form<2, 4, 4, 2, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
+    case 5: launch_i8_form<4, 2, 2, 5, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
+    default: launch_dl_shape<4, 1, 1, 5, OUT, 128>(A, B, xs, ws, bias, out, M, N, K, r, resid, s); break;
+    }
+}
+
 // K % 16 == 0 otherwise: the predicated register-staged kernel
 template <int OUT>
 static void dispatch(const int8_t* A, const int8_t* B, const float* xs, const float* ws, const void* bias,
-                     void* out, int M, int N, int K, hipStream_t s) {
+                     void* out, int M, int N, int K, const I8Plan* plan, void* part, hipStream_t s) {
+    if (plan) {
+        launch_i8_plan<OUT>(*plan, A, B, xs, ws, bias, out, M, N, K, {}, false, part, s);
+        return;
+    }
     if (K % kDlBK == 0) {
         launch_dl<OUT>(A, B, xs, ws, bias, out, M, N, K, {}, false, s);
         return;
@@ -562,7 +746,11 @@ static void dispatch(const int8_t* A, const int8_t* B, const float* xs, const fl
 }
 
 static void dispatch_resid(const int8_t* A, const int8_t* B, const float* xs, const float* ws, void* out, int M, int N,
-                           int K, Residual r, hipStream_t s) {
+                           int K, Residual r, const I8Plan* plan, void* part, hipStream_t s) {
+    if (plan) {
+        launch_i8_plan<WF_BF16>(*plan, A, B, xs, ws, nullptr, out, M, N, K, r, true, part, s);
+        return;
+    }
     if (K % kDlBK == 0) {
         launch_dl<WF_BF16>(A, B, xs, ws, nullptr, out, M, N, K, r, true, s);
         return;
@@ -577,24 +765,52 @@ static void dispatch_resid(const int8_t* A, const int8_t* B, const float* xs, co
     }
 }
 
+static int check_i8(const char* who, const int8_t* xq, const int8_t* wq, const float* xs, const float* ws,
+                    const void* out, int out_dt, int64_t M, int64_t N, int64_t K) {
+    if (M < 0 || N < 0 || K <= 0) { set_error("%s: M, N, K = %lld, %lld, %lld", who, (long long)M, (long long)N, (long long)K); return WF_EINVAL; }
+    if (M == 0 || N == 0) return WF_OK;
+    if (!xq || !wq || !xs || !ws || !out) { set_error("%s: null pointer", who); return WF_EINVAL; }
+    if (out_dt != WF_BF16 && out_dt != WF_F16) { set_error("%s: output dtype %d", who, out_dt); return WF_EUNSUPPORTED; }
+    if (K % 16 || !aligned(xq, 16) || !aligned(wq, 16)) {
+        set_error("%s: K %% 16 == 0 and 16-byte aligned operands are required", who);
+        return WF_EUNSUPPORTED;
+    }
+    if (M >= (1LL << 31) || N >= (1LL << 31) || M * N >= (1LL << 62)) {
+        set_error("%s: sizes beyond the kernels' 32-bit tile indices", who);
+        return WF_EUNSUPPORTED;
+    }
+    // int32 accumulation is exact when K * 128 * 128 < 2^31
+    if (K > 131071) { set_error("%s: K = %lld would overflow the int32 accumulator", who, (long long)K); return WF_EUNSUPPORTED; }
+    return WF_OK;
+}
+
+// the checks of the residual's operands, and `res` from them
+static int check_i8_residual(const char* who, const void* gate, const void* resid, int64_t M, int64_t rows_per_group,
+                             Residual* res) {
+    if (!gate || !resid) { set_error("%s: null pointer", who); return WF_EINVAL; }
+    if (M % rows_per_group) { set_error("%s: M is not a whole number of row groups", who); return WF_EUNSUPPORTED; }
+    // (a group of 2^31 rows or more holds them all)
+    *res = {static_cast<const uint16_t*>(gate), static_cast<const uint16_t*>(resid),
+            (int)std::min<int64_t>(rows_per_group, 0x7fffffff)};
+    return WF_OK;
+}
+
 }  // namespace wf
 
 extern "C" int wf_linear_i8_residual(const int8_t* xq, const int8_t* wq, const float* xs, const float* ws,
                                      const void* gate_bf16, const void* resid_bf16, void* out_bf16, int64_t M,
                                      int64_t N, int64_t K, int64_t rows_per_group, void* stream) {
     using namespace wf;
-    if (M < 0 || N < 0 || K <= 0 || rows_per_group <= 0) { set_error("wf_linear_i8_residual: bad sizes"); return WF_EINVAL; }
-    if (M == 0 || N == 0) return WF_OK;
-    if (!xq || !wq || !xs || !ws || !gate_bf16 || !resid_bf16 || !out_bf16) { set_error("wf_linear_i8_residual: null pointer"); return WF_EINVAL; }
-    if (K % 16 || !aligned(xq, 16) || !aligned(wq, 16)) {
-        set_error("wf_linear_i8_residual: K %% 16 == 0 and 16-byte aligned operands are required");
-        return WF_EUNSUPPORTED;
-    }
-    if (M % rows_per_group) { set_error("wf_linear_i8_residual: M is not a whole number of row groups"); return WF_EUNSUPPORTED; }
-    if (M >= (1LL << 31) || N >= (1LL << 31) || K > 131071) { set_error("wf_linear_i8_residual: sizes too large"); return WF_EUNSUPPORTED; }
-    Residual r{static_cast<const uint16_t*>(gate_bf16), static_cast<const uint16_t*>(resid_bf16), (int)rows_per_group};
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    dispatch_resid(xq, wq, xs, ws, out_bf16, (int)M, (int)N, (int)K, r, s);
+    if (rows_per_group <= 0) { set_error("wf_linear_i8_residual: bad sizes"); return WF_EINVAL; }
+    int rc = check_i8("wf_linear_i8_residual", xq, wq, xs, ws, out_bf16, WF_BF16, M, N, K);
+    if (rc != WF_OK || M == 0 || N == 0) return rc;
+    Residual r{};
+    rc = check_i8_residual("wf_linear_i8_residual", gate_bf16, resid_bf16, M, rows_per_group, &r);
+    if (rc != WF_OK) return rc;
+    const bool modelled = i8_modelled(M, N, K);
+    const I8Plan plan = modelled ? i8_plan(M, N, K, 0) : I8Plan{};
+    dispatch_resid(xq, wq, xs, ws, out_bf16, (int)M, (int)N, (int)K, r, modelled ? &plan : nullptr, nullptr,
+                   static_cast<hipStream_t>(stream));
     WF_LAUNCH_CHECK("wf_linear_i8_residual launch");
     return WF_OK;
 }
@@ -602,23 +818,54 @@ extern "C" int wf_linear_i8_residual(const int8_t* xq, const int8_t* wq, const f
 extern "C" int wf_linear_i8(const int8_t* xq, const int8_t* wq, const float* xs, const float* ws, const void* bias,
                             void* out, int out_dt, int64_t M, int64_t N, int64_t K, void* stream) {
     using namespace wf;
-    if (M < 0 || N < 0 || K <= 0) { set_error("wf_linear_i8: M, N, K = %lld, %lld, %lld", (long long)M, (long long)N, (long long)K); return WF_EINVAL; }
-    if (M == 0 || N == 0) return WF_OK;
-    if (!xq || !wq || !xs || !ws || !out) { set_error("wf_linear_i8: null pointer"); return WF_EINVAL; }
-    if (out_dt != WF_BF16 && out_dt != WF_F16) { set_error("wf_linear_i8: output dtype %d", out_dt); return WF_EUNSUPPORTED; }
-    if (K % 16 || !aligned(xq, 16) || !aligned(wq, 16)) {
-        set_error("wf_linear_i8: K %% 16 == 0 and 16-byte aligned operands are required");
-        return WF_EUNSUPPORTED;
-    }
-    if (M >= (1LL << 31) || N >= (1LL << 31) || K >= (1LL << 31) || M * N >= (1LL << 62)) {
-        set_error("wf_linear_i8: sizes beyond the kernels' 32-bit tile indices");
-        return WF_EUNSUPPORTED;
-    }
-    // int32 accumulation is exact when K * 128 * 128 < 2^31
-    if (K > 131071) { set_error("wf_linear_i8: K = %lld would overflow the int32 accumulator", (long long)K); return WF_EUNSUPPORTED; }
+    const int rc = check_i8("wf_linear_i8", xq, wq, xs, ws, out, out_dt, M, N, K);
+    if (rc != WF_OK || M == 0 || N == 0) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (out_dt == WF_BF16) dispatch<WF_BF16>(xq, wq, xs, ws, bias, out, (int)M, (int)N, (int)K, s);
-    else dispatch<WF_F16>(xq, wq, xs, ws, bias, out, (int)M, (int)N, (int)K, s);
+    const bool modelled = i8_modelled(M, N, K);
+    const I8Plan plan = modelled ? i8_plan(M, N, K, 0) : I8Plan{};
+    const I8Plan* p = modelled ? &plan : nullptr;
+    if (out_dt == WF_BF16) dispatch<WF_BF16>(xq, wq, xs, ws, bias, out, (int)M, (int)N, (int)K, p, nullptr, s);
+    else dispatch<WF_F16>(xq, wq, xs, ws, bias, out, (int)M, (int)N, (int)K, p, nullptr, s);
     WF_LAUNCH_CHECK("wf_linear_i8 launch");
+    return WF_OK;
+}
+
+extern "C" int wf_linear_i8_workspace(int64_t M, int64_t N, int64_t K, int64_t* bytes) {
+    using namespace wf;
+    if (!bytes) { set_error("wf_linear_i8_workspace: null out-pointer"); return WF_EINVAL; }
+    *bytes = 0;
+    if (M < 0 || N < 0 || K <= 0) { set_error("wf_linear_i8_workspace: M, N, K"); return WF_EINVAL; }
+    if (M > 0 && N > 0 && M < (1LL << 31) && N < (1LL << 31) && K <= 131071 && i8_modelled(M, N, K))
+        *bytes = i8_plan(M, N, K, INT64_MAX).part_bytes;
+    return WF_OK;
+}
+
+extern "C" int wf_linear_i8_ws(const int8_t* xq, const int8_t* wq, const float* xs, const float* ws, const void* bias,
+                               const void* gate_bf16, const void* resid_bf16, void* out, int out_dt, int64_t M,
+                               int64_t N, int64_t K, int64_t rows_per_group, void* workspace, int64_t workspace_bytes,
+                               void* stream) {
+    using namespace wf;
+    int rc = check_i8("wf_linear_i8_ws", xq, wq, xs, ws, out, out_dt, M, N, K);
+    const bool resid = gate_bf16 || resid_bf16;
+    if (rc == WF_OK && resid && (rows_per_group <= 0 || bias || out_dt != WF_BF16)) {
+        set_error("wf_linear_i8_ws: the residual form takes whole row groups, a bf16 output and no bias");
+        return WF_EINVAL;
+    }
+    if (rc != WF_OK || M == 0 || N == 0) return rc;
+    Residual r{};
+    if (resid && (rc = check_i8_residual("wf_linear_i8_ws", gate_bf16, resid_bf16, M, rows_per_group, &r)) != WF_OK) return rc;
+    const bool modelled = i8_modelled(M, N, K);
+    const I8Plan plan = modelled ? i8_plan(M, N, K, INT64_MAX) : I8Plan{};
+    if (plan.part_bytes > 0 && (!workspace || !aligned(workspace, 256) || workspace_bytes < plan.part_bytes)) {
+        set_error("wf_linear_i8_ws: a 256-byte aligned workspace of %lld bytes is needed (given %lld)",
+                  (long long)plan.part_bytes, (long long)workspace_bytes);
+        return WF_EINVAL;
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const I8Plan* p = modelled ? &plan : nullptr;
+    if (resid) dispatch_resid(xq, wq, xs, ws, out, (int)M, (int)N, (int)K, r, p, workspace, s);
+    else if (out_dt == WF_BF16) dispatch<WF_BF16>(xq, wq, xs, ws, bias, out, (int)M, (int)N, (int)K, p, workspace, s);
+    else dispatch<WF_F16>(xq, wq, xs, ws, bias, out, (int)M, (int)N, (int)K, p, workspace, s);
+    WF_LAUNCH_CHECK("wf_linear_i8_ws launch");
     return WF_OK;
 }

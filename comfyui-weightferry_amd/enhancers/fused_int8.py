@@ -14,8 +14,8 @@ What a call here computes, for a bf16 input x [m, k] and an int8 ConvRot weight 
 * an input may arrive *pending*: the block registered that the real input is op(marker) -- a scale-and-shift
   (``mod``), LayerNorm then scale-and-shift (``lnmod``), or GELU (``gelu``) -- and the layer receives ``marker``;
   the operation then runs inside the quantiser and the real input is never written;
-* the int8 GEMM with the scale epilogue (``wf_linear_i8``), or with the gated residual ``x_res + gate * out``
-  (``wf_linear_i8_residual``) when the block left its residual pending.
+* the int8 GEMM with the scale epilogue, or with the gated residual ``x_res + gate * out`` when the block left its
+  residual pending (``wf_linear_i8_ws``).
 
 The per-thread state lives in ``fused_state._tls``: ``qkv`` (the shared quantisation, a dict while ``_Overrides``
 is active), ``pre`` (the pending input), ``res`` (the pending residual). The names of this module's functions and
@@ -23,6 +23,7 @@ of those three fields are the reference's protocol between its block and its lin
 enhancers/fused_block.py); the eligibility rules follow enhancers/fused_int8.py:108-147.
 """
 import atexit
+import ctypes
 from collections import namedtuple
 
 import torch
@@ -58,29 +59,46 @@ def quantise_rows(x_2d, mode):
     return (x_q, x_s) if _native.check(rc, "wf_quant_rows_i8") else None
 
 
+_needs = {}                  # (m, n, k) -> the bytes wf_linear_i8_workspace gives
+
+
+def _workspace(m, n, k, dev):
+    """The workspace of an int8 GEMM of this shape (K-slice sums), or None where it needs none. A new tensor each call:
+    torch's allocator hands its memory on only to work queued later on this stream."""
+    need = _needs.get((m, n, k))
+    if need is None:
+        v = ctypes.c_int64()
+        _native.call("wf_linear_i8_workspace", m, n, k, ctypes.byref(v))
+        if len(_needs) > 4096:
+            _needs.clear()
+        need = _needs[m, n, k] = v.value
+    return torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+
+
+def _linear_i8(x_q, x_s, w_q, ws, bias, gate, resid, out, rows_per_gate):
+    """wf_linear_i8_ws; False when the library declines."""
+    m, k = x_q.shape
+    n, dev = w_q.shape[0], x_q.device
+    with _native.on_device(dev):
+        part = _workspace(m, n, k, dev)
+        rc = _native.lib().wf_linear_i8_ws(
+            x_q.data_ptr(), w_q.data_ptr(), x_s.data_ptr(), ws.data_ptr(), None if bias is None else bias.data_ptr(),
+            None if gate is None else gate.data_ptr(), None if resid is None else resid.data_ptr(), out.data_ptr(),
+            1 if out.dtype == torch.bfloat16 else 0, m, n, k, rows_per_gate, None if part is None else part.data_ptr(),
+            0 if part is None else part.numel(), _stream(dev))
+    return _native.check(rc, "wf_linear_i8")
+
+
 def gemm(x_q, x_s, w_q, ws, out_dtype=torch.bfloat16, bias=None):
     """out[m, n] = out_dtype((float(sum_k x_q[m, k] w_q[n, k]) * x_s[m]) * ws[n] (+ bias[n])), the sum exact in
     int32; None when the library declines."""
-    m, k = x_q.shape
-    n = w_q.shape[0]
-    dev = x_q.device
-    out = torch.empty((m, n), dtype=out_dtype, device=dev)
-    code = 1 if out_dtype == torch.bfloat16 else 0
-    with _native.on_device(dev):
-        rc = _native.lib().wf_linear_i8(x_q.data_ptr(), w_q.data_ptr(), x_s.data_ptr(), ws.data_ptr(),
-                                        None if bias is None else bias.data_ptr(), out.data_ptr(), code, m, n, k,
-                                        _stream(dev))
-    return out if _native.check(rc, "wf_linear_i8") else None
+    out = torch.empty((x_q.shape[0], w_q.shape[0]), dtype=out_dtype, device=x_q.device)
+    return out if _linear_i8(x_q, x_s, w_q, ws, bias, None, None, out, 1) else None
 
 
 def _gemm_residual(q, gate_2d, resid_2d, out_2d, rows_per_gate):
-    """wf_linear_i8_residual: out = bf16(resid + gate[row // rows_per_gate] * linear) over q's rows."""
-    with _native.on_device(q.device):
-        rc = _native.lib().wf_linear_i8_residual(q.x_q.data_ptr(), q.w_q.data_ptr(), q.x_s.data_ptr(),
-                                                 q.ws.data_ptr(), gate_2d.data_ptr(), resid_2d.data_ptr(),
-                                                 out_2d.data_ptr(), q.m, q.n, q.w_q.shape[1], rows_per_gate,
-                                                 _stream(q.device))
-    return _native.check(rc, "wf_linear_i8_residual")
+    """The residual form: out = bf16(resid + gate[row // rows_per_gate] * linear) over q's rows."""
+    return _linear_i8(q.x_q, q.x_s, q.w_q, q.ws, None, gate_2d, resid_2d, out_2d, rows_per_gate)
 
 
 # ------------------------------------------------------------------------------------- a direct entry point

@@ -101,6 +101,15 @@ int wf_linear_i8_residual(const int8_t* xq, const int8_t* wq, const float* xs, c
                           const void* resid_bf16, void* out_bf16, int64_t M, int64_t N, int64_t K,
                           int64_t rows_per_group, void* stream);
 
+/* Either form with a workspace, in which a product too small to fill the chip runs as K slices whose int32 sums are
+ * added afterwards (the same bits): gate and resid NULL for the plain form, both set for the residual one (then bias is
+ * NULL and out_dt WF_BF16). wf_linear_i8_workspace gives the bytes for a shape (0: none needed); the workspace is
+ * 256-byte aligned, need not be cleared and is free again when the call's work on the stream is done. */
+int wf_linear_i8_workspace(int64_t M, int64_t N, int64_t K, int64_t* bytes);
+int wf_linear_i8_ws(const int8_t* xq, const int8_t* wq, const float* xs, const float* ws, const void* bias,
+                    const void* gate_bf16, const void* resid_bf16, void* out, int out_dt, int64_t M, int64_t N,
+                    int64_t K, int64_t rows_per_group, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------------- fused dequant + bf16 GEMM
  * y[m, n] = bf16(sum_k x[m, k] * W[n, k] (+ bias[n])) with W given as GGUF K-quant blocks (qtype 12 Q4_K, 13 Q5_K, 14
  * Q6_K; [N, K] row-major in 256-value super-blocks, wq_bytes = N * K / 256 * block bytes; also qtype 8 Q8_0, 34 bytes

@@ -5,6 +5,8 @@ Quantiser: bf16 N(0, 1) rows at several widths (incl. the 14B-DiT width 5120), p
 largest value and rows built to hit rint ties. GEMM: ragged small shapes (tails in M, N and K) against the C oracle,
 and every workload shape (M in {1024, 4096, 16384}, K = 5120, N in {5120, 13824}) on sampled rows against an exact
 float64 accumulator with the epilogue in torch float32 (the same operations as the oracle's epilogue)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -394,3 +396,40 @@ def test_residual_runs_and_single_values(native, M, N, K, off):
     assert rc == 0, native.last_error()
     torch.cuda.synchronize()
     assert torch.equal(y.cpu().view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1000, 2048), (32, 5120, 5120), (33, 2040, 8192), (64, 1111, 4096), (100, 3000, 2560),
+                                   (129, 2048, 8192), (300, 1288, 5120), (520, 2048, 13824)])
+def test_gemm_in_slices_of_k(native, M, N, K):
+    # the K-slice form, rows around its 32-, 64- and 128-row tiles, widths that leave a partial last tile (1111: single
+    # values; the others: 16-byte runs), a last slice shorter than the others; plain, bias, float16 and residual
+    g = torch.Generator().manual_seed(M + N)
+    xq, wq = _rand_i8(g, (M, K)), _rand_i8(g, (N, K))
+    xs, ws = torch.rand(M, generator=g) * 0.05 + 1e-3, torch.rand(N, generator=g) * 0.002 + 1e-5
+    bias, resid = (torch.randn(s, generator=g).to(torch.bfloat16) for s in ((N,), (M, N)))
+    gate = torch.randn((1, N), generator=g).to(torch.bfloat16)
+    need = ctypes.c_int64()
+    assert native.lib().wf_linear_i8_workspace(M, N, K, ctypes.byref(need)) == 0 and need.value > 0
+    part = torch.full((need.value,), 0x5A, dtype=torch.uint8, device="cuda")
+    d = {k: v.cuda() for k, v in dict(xq=xq, wq=wq, xs=xs, ws=ws, bias=bias, gate=gate, resid=resid).items()}
+    # |acc| < 13824 * 127^2 < 2^28: exact in the float64 product, then one rounding to float32 as the kernel's
+    t = ((xq.double() @ wq.double().T).float() * xs[:, None]) * ws[None, :]
+
+    def run(dtype, **kw):
+        y = torch.empty((M, N), dtype=dtype, device="cuda")
+        p = {k: d[k].data_ptr() if kw.get(k) else None for k in ("bias", "gate", "resid")}
+        rc = native.lib().wf_linear_i8_ws(d["xq"].data_ptr(), d["wq"].data_ptr(), d["xs"].data_ptr(), d["ws"].data_ptr(),
+                                          p["bias"], p["gate"], p["resid"], y.data_ptr(), int(dtype == torch.bfloat16), M, N,
+                                          K, M, part.data_ptr(), part.numel(), native.stream_of(y.device))
+        assert rc == 0, native.last_error()
+        torch.cuda.synchronize()
+        return y.cpu().view(torch.int16)
+    b16 = t.to(torch.bfloat16)
+    for _ in range(2):                                            # the workspace is reused as it was left
+        assert torch.equal(run(torch.bfloat16), b16.view(torch.int16))
+    assert torch.equal(run(torch.bfloat16, bias=1), (t + bias.float()).to(torch.bfloat16).view(torch.int16))
+    assert torch.equal(run(torch.float16), t.to(torch.float16).view(torch.int16))
+    assert torch.equal(run(torch.bfloat16, gate=1, resid=1), torch.addcmul(resid, gate, b16).view(torch.int16))
+    assert native.lib().wf_linear_i8_ws(d["xq"].data_ptr(), d["wq"].data_ptr(), d["xs"].data_ptr(), d["ws"].data_ptr(), None,
+                                        None, None, part.data_ptr(), 1, M, N, K, 1, part.data_ptr(), need.value - 1,
+                                        None) == native.EINVAL      # refused before any launch
