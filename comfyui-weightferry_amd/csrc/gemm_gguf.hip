@@ -918,7 +918,7 @@ __global__ __launch_bounds__(64 * kSpWaves) void gemm_gguf_splitk(const uint16_t
 // Between the few-rows kernel (every workgroup reads its activation fragments from L2: too much traffic beyond 64
 // rows, and from 17-33 rows on the panel's split K already fills the chip better) and the tiled kernel (256 x 320
 // output tiles: 16-128 workgroups on 256 CUs below 2048 rows), a workgroup takes a panel: 128 weight rows (4 waves,
-// each two 16-row groups as in the few-rows kernel) against BM = 16 MT activation rows (MT = 2, 4 or 8), over a
+// each two 16-row groups as in the few-rows kernel) against BM = 16 MT activation rows (MT = 2 to 8), over a
 // slice of KS super-blocks of K. The activations stream through a two-buffer LDS ring, one
 // half super-block (BM rows x 256 bytes) per buffer -- 64 KiB at 128 rows, so two workgroups share a CU --, copied
 // by the load unit straight into LDS (buffer_load ... lds) one half ahead, 16-byte chunk c of row r at chunk
@@ -1373,8 +1373,8 @@ static int check_gguf(const char* who, const void* x_bf16, int64_t M, int64_t K,
     return WF_OK;
 }
 
-// Medium row counts: the panel kernel's plan. MT = 2 up to 32 rows, 4 up to 64, else 8 (128 activation rows per
-// panel); slices S so that NT x MTI x S >= 256 workgroups, at least two super-blocks each, and partial sums no larger
+// Medium row counts: the panel kernel's plan. Panels of up to 32 rows up to 32, 64 up to 64, else 128 (panel_plan has
+// the exact heights); slices S so that NT x MTI x S >= 256 workgroups, at least two super-blocks each, and partial sums no larger
 // than max_part bytes (0: one slice, no workspace). Up to 512 rows it beats the tiled kernel (Wan block, Q4_K, one
 // slice: 563 against 856 us at 128 rows, 684 against 887 at 512); from 1024 rows the tiled kernel's 256 x 320 tiles,
 // which dequantise each weight value once per 256 rows instead of once per 128, are faster (909 against 1334 us).
@@ -1409,12 +1409,22 @@ struct PanelPlan {
 // partial sums cost more than the second workgroup gains (Q4_K 303 against 289 at 256 rows).
 static int panel_target(int64_t M, int qtype) { return M > 384 || (qtype == 14 && M <= 128) ? 512 : 256; }
 
-static PanelPlan panel_plan(int64_t M, int64_t N, int64_t K, int64_t max_part, int qtype) {
+static PanelPlan panel_plan(int64_t M, int64_t N, int64_t K, int64_t max_part, int qtype, int mid_dt) {
     PanelPlan p{};
     // (Q8_0's raw bytes, 24 registers per row group and set against the K-quants' 12, leave 128-row panels short of
     // registers at two waves per SIMD: they spilled 60; its panels take 64 rows)
     p.mt = M <= 32 ? 2 : M <= 64 || qtype == 8 ? 4 : 8;
     p.mti = (int)((M + 16 * p.mt - 1) / (16 * p.mt));
+    // the lowest panels, in steps of 16 rows, that cover M in the same number of them (MID f16, the usual one: the
+    // others keep the three heights). A panel's MFMAs and fragment reads go with its height. Against 32-, 64- and
+    // 128-row panels, the Wan shapes and 2048 x 2048 (MI355X, bit-identical): Q4_K / Q5_K 1.13 times as fast at 77
+    // rows, 1.16 at 140, 1.04 at 100 and 300, Q8_0 1.03 at 40-90; Q6_K 1.15 at 77 and 140, 1.09 at 100 (5120 x 5120
+    // at 140 rows Q4_K 30.6 against 35.8 us, Q6_K 49.0 against 55.5). Q6_K's 48-row panels lost to 64-row ones (0.98)
+    // and its 80-row ones to 96-row ones (13824 x 5120 at 77 rows 69.3 against 59.7 us).
+    if (mid_dt == WF_F16) {
+        const int need = (int)((M + 16 * p.mti - 1) / (16 * p.mti));
+        p.mt = qtype == 14 && (need == 3 || need == 5) ? need + 1 : std::max(2, need);
+    }
     p.nt = (int)((N + kPnRows - 1) / kPnRows);
     const int nsb = (int)(K / 256);
     const int64_t tiles = (int64_t)p.nt * p.mti;
@@ -1448,21 +1458,32 @@ static void launch_panel_mt(const uint16_t* X, const uint8_t* W, const uint16_t*
     }
 }
 
+template <int QT, int MT>
+static void launch_panel_mid(int mid, const uint16_t* X, const uint8_t* W, const uint16_t* bias, uint16_t* Y, int M,
+                             int N, int K, const PanelPlan& p, void* ws, hipStream_t st) {
+    if (mid == WF_F16) launch_panel_mt<QT, WF_F16, MT>(X, W, bias, Y, M, N, K, p, ws, st);
+    else if (mid == WF_BF16) launch_panel_mt<QT, WF_BF16, MT>(X, W, bias, Y, M, N, K, p, ws, st);
+    else launch_panel_mt<QT, WF_F32, MT>(X, W, bias, Y, M, N, K, p, ws, st);
+}
+
+// (heights 3, 5, 6 and 7 are MID f16's alone, Q6_K has no 3 and 5, Q8_0 none above 4: panel_plan)
 template <int QT>
 static void launch_panel(int mid, const uint16_t* X, const uint8_t* W, const uint16_t* bias, uint16_t* Y, int M,
                          int N, int K, const PanelPlan& p, void* ws, hipStream_t st) {
-    if (p.mt == 2) {
-        if (mid == WF_F16) launch_panel_mt<QT, WF_F16, 2>(X, W, bias, Y, M, N, K, p, ws, st);
-        else if (mid == WF_BF16) launch_panel_mt<QT, WF_BF16, 2>(X, W, bias, Y, M, N, K, p, ws, st);
-        else launch_panel_mt<QT, WF_F32, 2>(X, W, bias, Y, M, N, K, p, ws, st);
-    } else if (p.mt == 4 || QT == 8) {                // (Q8_0: 64-row panels at most, panel_plan)
-        if (mid == WF_F16) launch_panel_mt<QT, WF_F16, 4>(X, W, bias, Y, M, N, K, p, ws, st);
-        else if (mid == WF_BF16) launch_panel_mt<QT, WF_BF16, 4>(X, W, bias, Y, M, N, K, p, ws, st);
-        else launch_panel_mt<QT, WF_F32, 4>(X, W, bias, Y, M, N, K, p, ws, st);
-    } else if constexpr (QT != 8) {
-        if (mid == WF_F16) launch_panel_mt<QT, WF_F16, 8>(X, W, bias, Y, M, N, K, p, ws, st);
-        else if (mid == WF_BF16) launch_panel_mt<QT, WF_BF16, 8>(X, W, bias, Y, M, N, K, p, ws, st);
-        else launch_panel_mt<QT, WF_F32, 8>(X, W, bias, Y, M, N, K, p, ws, st);
+    if (p.mt == 2) launch_panel_mid<QT, 2>(mid, X, W, bias, Y, M, N, K, p, ws, st);
+    else if (p.mt == 4 || (QT == 8 && p.mt > 4)) launch_panel_mid<QT, 4>(mid, X, W, bias, Y, M, N, K, p, ws, st);
+    else {
+        if constexpr (QT != 14) {
+            if (p.mt == 3) { launch_panel_mt<QT, WF_F16, 3>(X, W, bias, Y, M, N, K, p, ws, st); return; }
+        }
+        if constexpr (QT == 12 || QT == 13) {
+            if (p.mt == 5) { launch_panel_mt<QT, WF_F16, 5>(X, W, bias, Y, M, N, K, p, ws, st); return; }
+        }
+        if constexpr (QT != 8) {
+            if (p.mt == 6) launch_panel_mt<QT, WF_F16, 6>(X, W, bias, Y, M, N, K, p, ws, st);
+            else if (p.mt == 7) launch_panel_mt<QT, WF_F16, 7>(X, W, bias, Y, M, N, K, p, ws, st);
+            else launch_panel_mid<QT, 8>(mid, X, W, bias, Y, M, N, K, p, ws, st);
+        }
     }
 }
 
@@ -1485,7 +1506,7 @@ static void run_gguf(int qtype, int mid_dt, const void* x_bf16, const void* wq, 
     const uint16_t* B = static_cast<const uint16_t*>(bias_bf16);
     uint16_t* Y = static_cast<uint16_t*>(out_bf16);
     if (panel_takes(M)) {                             // without a workspace: one slice
-        run_gguf_panel(qtype, mid_dt, x_bf16, wq, bias_bf16, out_bf16, M, N, K, panel_plan(M, N, K, 0, qtype), nullptr,
+        run_gguf_panel(qtype, mid_dt, x_bf16, wq, bias_bf16, out_bf16, M, N, K, panel_plan(M, N, K, 0, qtype, mid_dt), nullptr,
                        s);
         return;
     }
@@ -1531,9 +1552,9 @@ extern "C" int wf_linear_gguf_workspace(int64_t M, int64_t N, int64_t K, int64_t
     // the format is not known here: the largest need over them (Q6_K's panels take more slices up to 128 rows)
     if (split_takes(M, N, K)) *bytes = split_plan(M, N, K).bytes();
     else if (panel_takes_ws(M, N, K)) {
-        const int64_t part = std::max({panel_plan(M, N, K, INT64_MAX, 12).part_bytes,
-                                       panel_plan(M, N, K, INT64_MAX, 14).part_bytes,
-                                       panel_plan(M, N, K, INT64_MAX, 8).part_bytes});
+        const int64_t part = std::max({panel_plan(M, N, K, INT64_MAX, 12, WF_F16).part_bytes,
+                                       panel_plan(M, N, K, INT64_MAX, 14, WF_F16).part_bytes,
+                                       panel_plan(M, N, K, INT64_MAX, 8, WF_F16).part_bytes});
         if (part > 0) *bytes = kSplitCounterBytes + part;   // the split form's counters stay untouched
     }
     return WF_OK;
@@ -1547,18 +1568,18 @@ extern "C" int wf_linear_gguf_ws(const void* x_bf16, int64_t M, int64_t K, const
     if (rc != WF_OK || M == 0 || N == 0) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     // Q8_0 up to 64 rows: the whole-rows or few-rows form (no workspace) unless the panel form's rule below takes it
-    if (qtype == 8 && M <= 64 && !(panel_takes_ws(M, N, K) && panel_plan(M, N, K, INT64_MAX, 8).s > 1)) {
+    if (qtype == 8 && M <= 64 && !(panel_takes_ws(M, N, K) && panel_plan(M, N, K, INT64_MAX, 8, mid_dt).s > 1)) {
         run_gguf_q8(mid_dt, x_bf16, wq, bias_bf16, out_bf16, (int)M, (int)N, (int)K, s);
         WF_LAUNCH_CHECK("wf_linear_gguf_ws launch");
         return WF_OK;
     }
     // up to 64 rows the panel form runs only in more than one slice (in one, the few-rows kernel is faster)
     const bool panel = !split_takes(M, N, K) && panel_takes_ws(M, N, K) &&
-                       (panel_takes(M) || panel_plan(M, N, K, INT64_MAX, qtype).s > 1);
+                       (panel_takes(M) || panel_plan(M, N, K, INT64_MAX, qtype, mid_dt).s > 1);
     if (panel) {
         // the panel form's partial sums go past the split form's counters, which must stay zero between calls (one
         // workspace serves calls of every shape and form on a stream)
-        const PanelPlan p = panel_plan(M, N, K, INT64_MAX, qtype);
+        const PanelPlan p = panel_plan(M, N, K, INT64_MAX, qtype, mid_dt);
         void* part = nullptr;
         if (p.part_bytes > 0) {
             const int64_t need = kSplitCounterBytes + p.part_bytes;
@@ -1636,16 +1657,16 @@ extern "C" int wf_linear_gguf_noalloc(const void* x_bf16, int64_t M, int64_t K, 
     hipStream_t s = static_cast<hipStream_t>(stream);
     // Q8_0 up to 64 rows: the whole-rows or few-rows form (no scratch) unless the panel form's rule below takes it
     if (qtype == 8 && M <= 64 &&
-        !(panel_takes_ws(M, N, K) && panel_plan(M, N, K, kScratchBytes - kSplitCounterBytes, 8).s > 1)) {
+        !(panel_takes_ws(M, N, K) && panel_plan(M, N, K, kScratchBytes - kSplitCounterBytes, 8, mid_dt).s > 1)) {
         run_gguf_q8(mid_dt, x_bf16, wq, bias_bf16, out_bf16, (int)M, (int)N, (int)K, s);
         WF_LAUNCH_CHECK("wf_linear_gguf_noalloc launch");
         return WF_OK;
     }
     // (up to 64 rows only when the scratch holds more than one slice: in one slice the few-rows kernel is faster)
     if (!split_takes(M, N, K) && panel_takes_ws(M, N, K) &&
-        (panel_takes(M) || panel_plan(M, N, K, kScratchBytes - kSplitCounterBytes, qtype).s > 1)) {
+        (panel_takes(M) || panel_plan(M, N, K, kScratchBytes - kSplitCounterBytes, qtype, mid_dt).s > 1)) {
         // the panel form's partial sums in the scratch array, as many slices as fit there
-        const PanelPlan p = panel_plan(M, N, K, kScratchBytes - kSplitCounterBytes, qtype);
+        const PanelPlan p = panel_plan(M, N, K, kScratchBytes - kSplitCounterBytes, qtype, mid_dt);
         void* part = nullptr;
         if (p.part_bytes > 0) {
             void* ws = nullptr;

@@ -461,3 +461,20 @@ def test_fused_linear_input_layouts(native, qtype, rows):
     assert fg.fused_linear(xd, torch.from_numpy(raw), qtype, (N, K), bias=bd) is None
     # nor is a 0-dimensional x (no row of K values)
     assert fg.fused_linear(xd[0, 0], rd, qtype, (N, K)) is None
+
+
+@pytest.mark.parametrize("qtype", [12, 13, 14, 8])
+def test_panel_heights(native, qtype):
+    # every panel height the plan uses (16 rows a step: 3 to 8, Q8_0 up to 4; one to three panels), at its last whole row,
+    # one row less and one more; 304 columns leave a partial 128-row weight panel, 10 super-blocks two slices or more
+    N, K = 304, 2560
+    raw = encode.random_blocks(qtype, nblocks(qtype, N, K), seed=qtype, family="normal")
+    w, rd = weight_bf16(raw, qtype, 0, N, K), torch.from_numpy(raw).cuda()
+    g = torch.Generator().manual_seed(qtype)
+    rows = (33, 48, 49, 66, 80, 81, 95, 96, 97, 112, 113, 129, 160, 161, 192, 224, 225, 257, 288, 336)
+    x = torch.randn((max(rows), K), generator=g).to(torch.bfloat16)
+    for M in rows:
+        print(f"case panel height qtype={qtype} M={M}", flush=True)
+        y, _, need = fused_ws(native, x[:M].cuda(), rd, qtype, N)
+        assert need > 0
+        check(y, x[:M], w)
