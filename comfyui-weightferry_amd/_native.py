@@ -192,13 +192,15 @@ def stream_wait(stream, event):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)   # without the initialisation check
 _no_guard = contextlib.nullcontext()
 
 
 def on_device(device):
     """``torch.cuda.device(device)`` when ``device`` is not the current device, else a no-op context: the library's
     kernels run on the current device, and the guard costs a few microseconds per call when it changes nothing."""
-    if device.index is None or device.index == torch.cuda.current_device():
+    index = device.index
+    if index is None or index == _current():
         return _no_guard
     return torch.cuda.device(device)
 
