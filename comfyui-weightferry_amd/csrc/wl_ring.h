@@ -174,15 +174,12 @@ __device__ __forceinline__ void wl_store_tile(uint16_t* ot, uint16_t* Y, int M, 
                 if (m < M && n < N) *reinterpret_cast<uint4*>(Y + (int64_t)m * N + n) = fin.run(v, f[it], m, n);
             }
         } else {
-            for (int it = 0; it < NIT; it++) {
-                const int q = it * 64 + lane, r = q / RUNS, c = q % RUNS;
-                const int m = mi + r;
-                if (m >= M) continue;
-                const uint16_t* row = ot + r * TC + 8 * c;
-                for (int e = 0; e < 8; e++) {
-                    const int n = nw + 8 * c + e;
-                    if (n < N) Y[(int64_t)m * N + n] = fin.one(row[e], m, n);
-                }
+            // 64 consecutive values a store (a lane that stored 8 of its own wrote 2 bytes in every 16: int8 4096 x 5119 x
+            // 5120 112 us against 96, 640 x 8885 x 1792 31.4 against 22.3; bf16 4096 x 5119 x 5120 181 against 165)
+            for (int it = 0; it < 32 * TC / 64; it++) {
+                const int q = it * 64 + lane, m = mi + q / TC, n = nw + q % TC;
+                const uint16_t v = ot[q];
+                if (m < M && n < N) Y[(int64_t)m * N + n] = fin.one(v, m, n);
             }
         }
     }
