@@ -9,6 +9,7 @@
 // and the pipeline are described at gemm_gguf_dl below.
 
 #include <algorithm>
+#include <tuple>
 #include <cstdint>
 #include <mutex>
 #include <type_traits>
@@ -1374,7 +1375,7 @@ static int check_gguf(const char* who, const void* x_bf16, int64_t M, int64_t K,
 }
 
 // Medium row counts: the panel kernel's plan. Panels of up to 32 rows up to 32, 64 up to 64, else 128 (panel_plan has
-// the exact heights); slices S so that NT x MTI x S >= 256 workgroups, at least two super-blocks each, and partial sums no larger
+// the exact heights); slices S by the modelled time, at least two super-blocks each, and partial sums no larger
 // than max_part bytes (0: one slice, no workspace). Up to 512 rows it beats the tiled kernel (Wan block, Q4_K, one
 // slice: 563 against 856 us at 128 rows, 684 against 887 at 512); from 1024 rows the tiled kernel's 256 x 320 tiles,
 // which dequantise each weight value once per 256 rows instead of once per 128, are faster (909 against 1334 us).
@@ -1403,11 +1404,20 @@ struct PanelPlan {
     int64_t part_bytes;
 };
 
-// Workgroups the slices aim for: 256 (one per CU), or 512 (two per CU, which the 64 KiB ring allows) where that
-// measured faster on MI355X (Wan shapes, warmed, with the workspace): from 385 rows (Q4_K block at 512 rows 473
-// against 495 us, Q6_K 739 against 818) and for Q6_K up to 128 rows (254 against 268 at 128); elsewhere the extra
-// partial sums cost more than the second workgroup gains (Q4_K 303 against 289 at 256 rows).
-static int panel_target(int64_t M, int qtype) { return M > 384 || (qtype == 14 && M <= 128) ? 512 : 256; }
+// Modelled ns of the panel form in s slices of ks super-blocks over `tiles` panels: a super-block costs its dequantisation
+// and, per 16 activation rows, its MFMAs; two workgroups share a CU in 1.58 times the time of one, three take 2.5 and
+// four 2.9 times; each slice's partial sums pass through memory once each way. Fitted to 432 measurements (Q4_K, Q6_K,
+// Q8_0; the Wan shapes and 2048 x 2048 at 40-400 rows, cold weights, MI355X; 6 % rms). Aiming for 256 workgroups (512
+// above 384 rows and for Q6_K up to 128) leaves a few CUs with one more than the others. The plan aims elsewhere where
+// that is modelled 8 % faster and slices keep three super-blocks (two were slower than modelled): 7 % on average over
+// those measurements, none slower: Q4_K 5120 x 5120 at 256 rows 33.2 against 37.3 us, Q6_K 5120 x 13824 at 300 rows 127
+// against 157, Q8_0 5120 x 13824 at 256 rows 92 against 124.
+static int64_t panel_time(int64_t tiles, int64_t s, int64_t ks, int mt, int64_t outputs, int qtype) {
+    const int64_t block = qtype == 14 ? 2252 + 368 * mt : qtype == 8 ? 2324 + 101 * mt : 1371 + 194 * mt;
+    const int64_t turns = (tiles * s + 255) / 256;
+    const int64_t share = turns <= 1 ? 1000 : turns == 2 ? 1577 : turns == 3 ? 2497 : 732 * turns;
+    return ks * block * share / 1000 + (s > 1 ? s * outputs * 1542 / 1000000 : 0);
+}
 
 static PanelPlan panel_plan(int64_t M, int64_t N, int64_t K, int64_t max_part, int qtype, int mid_dt) {
     PanelPlan p{};
@@ -1421,18 +1431,26 @@ static PanelPlan panel_plan(int64_t M, int64_t N, int64_t K, int64_t max_part, i
     // rows, 1.16 at 140, 1.04 at 100 and 300, Q8_0 1.03 at 40-90; Q6_K 1.15 at 77 and 140, 1.09 at 100 (5120 x 5120
     // at 140 rows Q4_K 30.6 against 35.8 us, Q6_K 49.0 against 55.5). Q6_K's 48-row panels lost to 64-row ones (0.98)
     // and its 80-row ones to 96-row ones (13824 x 5120 at 77 rows 69.3 against 59.7 us).
-    if (mid_dt == WF_F16) {
-        const int need = (int)((M + 16 * p.mti - 1) / (16 * p.mti));
-        p.mt = qtype == 14 && (need == 3 || need == 5) ? need + 1 : std::max(2, need);
-    }
+    const int need = (int)((M + 16 * p.mti - 1) / (16 * p.mti));
+    // (the slices go by this height for every MID: the workspace query knows no MID)
+    const int height = qtype == 14 && (need == 3 || need == 5) ? need + 1 : std::max(2, need);
+    if (mid_dt == WF_F16) p.mt = height;
     p.nt = (int)((N + kPnRows - 1) / kPnRows);
     const int nsb = (int)(K / 256);
     const int64_t tiles = (int64_t)p.nt * p.mti;
-    const int64_t target = panel_target(M, qtype);
-    int s = (int)std::min<int64_t>((target + tiles - 1) / tiles, std::max(1, nsb / 2));
-    while (s > 1 && (int64_t)s * M * N * 4 > max_part) s--;
-    p.ks = (nsb + s - 1) / s;
-    p.s = (nsb + p.ks - 1) / p.ks;
+    auto slices = [&](int64_t target) {               // (slices, super-blocks of each) for `target` workgroups
+        int s = (int)std::min<int64_t>((target + tiles - 1) / tiles, std::max(1, nsb / 2));
+        while (s > 1 && (int64_t)s * M * N * 4 > max_part) s--;
+        const int ks = (nsb + s - 1) / s;
+        return std::make_pair((nsb + ks - 1) / ks, ks);
+    };
+    std::tie(p.s, p.ks) = slices(M > 384 || (qtype == 14 && M <= 128) ? 512 : 256);
+    int64_t best = panel_time(tiles, p.s, p.ks, height, M * N, qtype) * 92 / 100;
+    for (int64_t target : {384, 512, 768}) {
+        const auto [s, ks] = slices(target);
+        const int64_t t = panel_time(tiles, s, ks, height, M * N, qtype);
+        if (ks >= 3 && t < best) { best = t; p.s = s; p.ks = ks; }
+    }
     p.part_bytes = p.s > 1 ? (int64_t)p.s * M * N * 4 : 0;
     return p;
 }
