@@ -108,8 +108,8 @@ def fused_linear(x, data, qtype, oshape, bias=None, mid_dtype=None):
 #     415 / 421 (Q6_K 607 against 413 at 320) -- except the wide ffn_up (n_out > k: 13824 x 5120, 102 against 85 µs
 #     at 320 rows, 324 panels on 256 CUs), which keeps the two-step flow above 256 rows; Q4_K up to 512 rows (with
 #     512 workgroups of K slices there): 5120 x 5120 58 against 61 µs at 512 rows, 5120 x 13824 122 against 137;
-#   * above that the two-step flow is faster: Q5_K 515 / 524 against 467 / 490 µs per block at 448 / 512 rows, Q6_K
-#     737 against 491 at 512; Q5_K 1.80 against 1.72 ms at 4096; at 8192 the tiled form wins only 5120 x 5120, by
+#   * above that the two-step flow is faster: Q6_K 737 against 491 µs per block at 512 rows (Q5_K see prefer_slices);
+#     Q5_K 1.80 against 1.72 ms at 4096; at 8192 the tiled form wins only 5120 x 5120, by
 #     5 % (Q4_K).
 # mode "fused" still takes the tiled form at any row count.
 FEW_ROWS = 64
@@ -127,6 +127,16 @@ def prefer_fused(rows, qtype, n_out, k):
     if n_out > k:
         limit = min(limit, 256)
     return rows <= limit
+
+
+# Q5_K at 385-512 rows, outputs no wider than K: with the panel form's K slices chosen by time the fused kernel beats the
+# two-step flow there too (us, cold weights, MI355X): 5120 x 5120 51.6 / 54.3 against 60.9 / 61.6 at 385 / 512 rows,
+# 5120 x 13824 113.7 against 142.4 and 2048 x 2048 23.1 against 28.6 at 512; the closest, 8192 x 9216, 114.3 / 128.6
+# against 119.5 / 123.7 at 400 / 512. Q6_K above 256 rows stays slower on most shapes (5120 x 5120 at 300 rows 52.7
+# against 47.4).
+def prefer_slices(rows, qtype, n_out, k):
+    """mode "auto" beyond ``prefer_fused``: True where the panel form in K slices is the faster one."""
+    return qtype == 13 and PANEL_ROWS[13] < rows <= 512 and n_out <= k
 
 
 # The two-step flow's GEMM: the library's wf_linear_bf16 (whole 128-byte lines through two LDS stage buffers, 256 x 320
@@ -173,7 +183,9 @@ def linear(x, data, qtype, oshape, bias=None, mid_dtype=None, mode="auto"):
     (wf_linear_bf16 where ``hand_gemm`` says it is the faster one, else torch.nn.functional.linear)."""
     rows = x.numel() // max(1, x.shape[-1]) if x.dim() else 0
     if mode == "auto":
-        mode = "fused" if prefer_fused(rows, qtype, oshape[0], oshape[1]) else "dequant"
+        n_out, k = oshape[0], oshape[1]
+        fused = prefer_fused(rows, qtype, n_out, k) or prefer_slices(rows, qtype, n_out, k)
+        mode = "fused" if fused else "dequant"
     if mode == "fused":
         y = fused_linear(x, data, qtype, oshape, bias, mid_dtype)
         if y is not None:

@@ -51,6 +51,13 @@ def test_prefer_fused_rule():
             assert not fg.prefer_fused(rows, q, 5120, 5120) and not fg.prefer_fused(rows, q, 5120, 13824)
 
 
+def test_prefer_slices_rule():
+    for rows in (385, 512):
+        assert fg.prefer_slices(rows, 13, 5120, 5120) and not fg.prefer_slices(rows, 13, 13824, 5120)
+        assert not fg.prefer_slices(rows, 14, 5120, 5120)
+    assert not fg.prefer_slices(384, 13, 5120, 5120) and not fg.prefer_slices(513, 13, 5120, 5120)
+
+
 def test_auto_routes_by_rows(monkeypatch):
     calls = []
 
