@@ -424,11 +424,7 @@ __global__ __launch_bounds__(64 * VM * VN) void gemm_i8_dl(const int8_t* __restr
                 *reinterpret_cast<uint4*>(Y + (int64_t)m * N + n) = fin.run(v, fin.prefetch(m, n), m, n);
         }
     } else {
-        for (int it = 0; it < TR * TC / 64; it++) {        // 64 consecutive values a store
-            const int q = it * 64 + lane, m = mw + q / TC, n = nw + q % TC;
-            const uint16_t v = ot[q];
-            if (m < M && n < N) Y[(int64_t)m * N + n] = fin.one(v, m, n);
-        }
+        store_values<TC, TR>(ot, Y, M, N, mw, nw, lane, fin);
     }
 }
 

@@ -138,6 +138,35 @@ struct StoreAsIs {
     __device__ __forceinline__ uint16_t one(uint16_t v, int, int) const { return v; }
 };
 
+// Rows [m0, m0 + ROWS) x columns [n0, n0 + TC) of Y from the wave's finished 16-bit values in LDS (row-major, TC a row),
+// for outputs whose rows are not whole aligned 16-byte runs: 64 consecutive values a store (a lane that stores 8 of its
+// own writes 2 bytes in every 16). Rows past M are not walked, and eight stores' LDS reads, and what fin loads for them,
+// are in flight together; one after another over every row they cost few rows more than the wider stores give. us, lane by
+// lane / one after another / here: int8 4096 x 5119 x 5120 115 / 98 / 97, 8 x 2607 x 3136 17.5 / 20.2 / 17.4, 300 x 3001 x
+// 704 11.5 / 12.8 / 11.3; with the residual 26 x 12332 x 2624 36.0 / 39.5 / 28.0, 1500 x 2047 x 4096 46.7 / 51.1 / 34.5;
+// bf16 4096 x 5119 x 5120 184 / 166 / 165, 5 x 6297 x 8192 75.4 / 78.0 / 75.1.
+template <int TC, int ROWS, typename Fin>
+__device__ __forceinline__ void store_values(const uint16_t* ot, uint16_t* Y, int M, int N, int m0, int n0, int lane,
+                                             const Fin& fin) {
+    static_assert(ROWS * TC % 512 == 0, "whole groups of eight stores");
+    const int stores = n0 < N ? (min(M - m0, ROWS) * TC + 63) / 64 : 0;
+    for (int it = 0; it < stores; it += 8) {
+        uint16_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = ot[(it + u) * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {                      // (whatever fin loads, before a store could hold it up)
+            const int q = (it + u) * 64 + lane;
+            v[u] = fin.one(v[u], min(m0 + q / TC, M - 1), min(n0 + q % TC, N - 1));
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int q = (it + u) * 64 + lane, m = m0 + q / TC, n = n0 + q % TC;
+            if (m < M && n < N) Y[(int64_t)m * N + n] = v[u];
+        }
+    }
+}
+
 // Stores the wave's WM * 32 x WN * 32 output tile at rows mw.., columns nw.. of Y [M, N] (16-bit values), 32 rows at
 // a time through its LDS region ot: bits(i, j, e) gives the output bits of accumulator element e of MFMA tile (i, j)
 // (row mw + 32 i + 8 (e / 4) + 4 (lane / 32) + e % 4, column nw + 32 j + lane % 32), fin's run() or one() the value
@@ -174,13 +203,7 @@ __device__ __forceinline__ void wl_store_tile(uint16_t* ot, uint16_t* Y, int M, 
                 if (m < M && n < N) *reinterpret_cast<uint4*>(Y + (int64_t)m * N + n) = fin.run(v, f[it], m, n);
             }
         } else {
-            // 64 consecutive values a store (a lane that stored 8 of its own wrote 2 bytes in every 16: int8 4096 x 5119 x
-            // 5120 112 us against 96, 640 x 8885 x 1792 31.4 against 22.3; bf16 4096 x 5119 x 5120 181 against 165)
-            for (int it = 0; it < 32 * TC / 64; it++) {
-                const int q = it * 64 + lane, m = mi + q / TC, n = nw + q % TC;
-                const uint16_t v = ot[q];
-                if (m < M && n < N) Y[(int64_t)m * N + n] = fin.one(v, m, n);
-            }
+            store_values<TC, 32>(ot, Y, M, N, mi, nw, lane, fin);
         }
     }
 }

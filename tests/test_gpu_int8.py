@@ -433,3 +433,32 @@ def test_gemm_in_slices_of_k(native, M, N, K):
     assert native.lib().wf_linear_i8_ws(d["xq"].data_ptr(), d["wq"].data_ptr(), d["xs"].data_ptr(), d["ws"].data_ptr(), None,
                                         None, None, part.data_ptr(), 1, M, N, K, 1, part.data_ptr(), need.value - 1,
                                         None) == native.EINVAL      # refused before any launch
+
+
+@pytest.mark.parametrize("K", [192, 256])
+@pytest.mark.parametrize("M,N", [(1, 1), (3, 161), (17, 321), (34, 1003), (130, 37), (260, 333)])
+def test_odd_widths_store_their_rows_only(native, M, N, K):
+    # single values go out in groups of eight stores of 64 (both rings): widths that end inside a group, rows that end
+    # inside a wave's 32 and waves without any; nothing is written past the last value
+    g = torch.Generator().manual_seed(M * N + K)
+    xq, wq = _rand_i8(g, (M, K)), _rand_i8(g, (N, K))
+    xs, ws = torch.rand(M, generator=g) * 0.05 + 1e-3, torch.rand(N, generator=g) * 0.002 + 1e-5
+    G = 2 if M % 2 == 0 else 1
+    gate, resid = torch.randn((G, N), generator=g).to(torch.bfloat16), torch.randn((M, N), generator=g).to(torch.bfloat16)
+    t = (((xq.double() @ wq.double().T).float() * xs[:, None]) * ws[None, :]).to(torch.bfloat16)
+    d = [v.cuda() for v in (xq, wq, xs, ws, gate, resid)]
+    for residual in (False, True):
+        y = torch.full((M * N + 64,), -7.0, dtype=torch.bfloat16, device="cuda")
+        if residual:
+            ref = torch.addcmul(resid, gate.repeat_interleave(M // G, 0), t)
+            rc = native.lib().wf_linear_i8_residual(*[v.data_ptr() for v in d], y.data_ptr(), M, N, K, M // G,
+                                                    native.stream_of(y.device))
+        else:
+            ref = t
+            rc = native.lib().wf_linear_i8(*[v.data_ptr() for v in d[:4]], None, y.data_ptr(), 1, M, N, K,
+                                           native.stream_of(y.device))
+        assert rc == 0, native.last_error()
+        torch.cuda.synchronize()
+        got = y.cpu()
+        assert torch.equal(got[:M * N].view(M, N).view(torch.int16), ref.view(torch.int16)), residual
+        assert bool((got[M * N:] == -7.0).all())
