@@ -303,6 +303,8 @@ constexpr uint32_t kGeluExp = 109, kGeluEntries = 24 * 128, kGeluFirst = kGeluEx
 // and after, bit-identical: 16384 x 5120 67-69 and 51-53 us (4.9 TB/s), 4096 x 13824 53 and 39; GELU 5152 x 8192 48-49
 // and 40-42 (its table read from LDS instead of the L2), LayerNorm 5152 x 2048 24.1 and 18.5, 4096 x 8192 96 and 51
 // (its statistics had an IEEE division per value); scale-and-shift 4096 x 5120 24.8 and 24.2.
+//
+// PRE 4 is GELU with every value read from the whole table in memory, one turn per wave (gelu_in_lds says where).
 template <int NP, int PRE, int W>
 __global__ __launch_bounds__(256) void quant_convrot(const uint16_t* __restrict__ x, int64_t M, int K,
                                                      int8_t* __restrict__ xq, float* __restrict__ xs, PreArgs pa) {
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(256) void quant_convrot(const uint16_t* __restrict_
     for (int turn = 0;; turn ^= 1) {
         float mu = 0.0f, rstd = 0.0f;
         const uint16_t *sr = nullptr, *hr = nullptr;
-        if constexpr (PRE >= 2) {
+        if constexpr (PRE == 2 || PRE == 3) {
             // (32-bit division where it fits: the 64-bit one is a long sequence)
             const int64_t grp = M < (1LL << 31) && pa.rows_per_group < (1LL << 31)
                                     ? (int64_t)((uint32_t)row / (uint32_t)pa.rows_per_group)
@@ -390,7 +392,12 @@ __global__ __launch_bounds__(256) void quant_convrot(const uint16_t* __restrict_
         for (int p = 0; p < NP; p++) {
             uint32_t u[8] = {raw[p][0].x, raw[p][0].y, raw[p][0].z, raw[p][0].w,
                              raw[p][1].x, raw[p][1].y, raw[p][1].z, raw[p][1].w};
-            if constexpr (PRE == 1) {
+            if constexpr (PRE == 4) {
+                if (live(p)) {
+#pragma unroll
+                    for (int h = 0; h < 8; h++) u[h] = pa.s[u[h] & 0xffffu] | ((uint32_t)pa.s[u[h] >> 16] << 16);
+                }
+            } else if constexpr (PRE == 1) {
                 if (live(p)) {
                     // |bits| of the pairs' members; all 16 in the LDS part of the table, or value by value
                     uint32_t lo = 0xffffffffu, hi = 0;
@@ -411,7 +418,7 @@ __global__ __launch_bounds__(256) void quant_convrot(const uint16_t* __restrict_
                             u[h] = pa.s[u[h] & 0xffffu] | ((uint32_t)pa.s[u[h] >> 16] << 16);
                     }
                 }
-            } else if constexpr (PRE >= 2) {
+            } else if constexpr (PRE == 2 || PRE == 3) {
                 load_mod(sr, hr, p + 1);
                 if (live(p)) {
                     const uint4 s0 = sh[p & 1][0], s1 = sh[p & 1][1], h0 = sh[p & 1][2], h1 = sh[p & 1][3];
@@ -521,6 +528,15 @@ static void launch_convrot_pre(const uint16_t* x, int64_t M, int K, int8_t* xq, 
     quant_convrot<NP, PRE, W><<<dim3((unsigned)grid), 256, 0, s>>>(x, M, K, xq, xs, pa);
 }
 
+// GELU from the table in LDS, or from memory. Filling it costs every workgroup 12 KiB of loads and a barrier before its
+// first row, which narrow rows do not earn back: (us, memory against LDS, MI355X) 256 values 64 rows 3.9 and 4.4, 8192
+// rows 8.3 and 9.5; 512 values 1024 rows 4.0 and 4.4; 1024 values 512 rows 4.1 and 4.3, but 2048 rows 5.3 and 5.0; 1280
+// values 65536 rows 97 and 105 (a turn of four rows is short), 16384 rows 30.5 and 29.6; from 1536 values on LDS wins at
+// every row count (2048 values: 64 rows 6.1 and 5.6, 4096 rows 13.2 and 9.8).
+static bool gelu_in_lds(int64_t M, int K) {
+    return K >= 1536 || (K > 1024 && M <= 16384) || (K == 1024 && M > 1024);
+}
+
 template <int PRE>
 static void launch_convrot(const uint16_t* x, int64_t M, int K, int8_t* xq, float* xs, const PreArgs& pa,
                            hipStream_t s) {
@@ -620,7 +636,9 @@ extern "C" int wf_quant_rows_i8_pre(const void* x_bf16, int64_t M, int64_t K, in
                      rows_per_group > 0 ? rows_per_group : 1, eps};
     const int k = (int)K;
     if (pre == 0) launch_convrot<0>(xp, M, k, xq, xs, pa, s);
-    else if (pre == 1) launch_convrot<1>(xp, M, k, xq, xs, pa, s);
+    else if (pre == 1 && gelu_in_lds(M, k)) launch_convrot<1>(xp, M, k, xq, xs, pa, s);
+    else if (pre == 1 && k <= 1024) launch_convrot_pre<1, 4, 1>(xp, M, k, xq, xs, pa, s);
+    else if (pre == 1) launch_convrot_pre<2, 4, 1>(xp, M, k, xq, xs, pa, s);      // (1280 values, many rows)
     else if (pre == 2) launch_convrot<2>(xp, M, k, xq, xs, pa, s);
     else launch_convrot<3>(xp, M, k, xq, xs, pa, s);
     WF_LAUNCH_CHECK("wf_quant_rows_i8_pre launch");

@@ -462,3 +462,20 @@ def test_odd_widths_store_their_rows_only(native, M, N, K):
         got = y.cpu()
         assert torch.equal(got[:M * N].view(M, N).view(torch.int16), ref.view(torch.int16)), residual
         assert bool((got[M * N:] == -7.0).all())
+
+
+@pytest.mark.parametrize("M,K", [(1, 256), (4099, 512), (3, 768), (1024, 1024), (1025, 1024), (5, 1280), (16385, 1280),
+                                 (2, 1536)])
+def test_gelu_table_in_lds_or_memory(native, M, K):
+    # both sides of the rule that reads the table from memory (narrow rows) or fills it into LDS, with every kind of value
+    # the LDS part leaves out in the first and the last row
+    g = torch.Generator().manual_seed(M + K)
+    x = (torch.randn((M, K), generator=g) * 1.5).to(torch.bfloat16)
+    odd = torch.tensor([0.0, -0.0, 1e-6, -3e-6, 64.0, -64.0, 3e4, -1e-38]).to(torch.bfloat16)
+    x[0], x[M - 1] = odd[torch.arange(K) % 8], odd[torch.arange(K) % 8]
+    table, tbits = _gelu_table_bits()
+    xq, xs = gpu_quant_pre(native, x.cuda(), 1, table.cuda())
+    rows = torch.unique(torch.cat([torch.arange(min(M, 40)), torch.arange(max(0, M - 40), M)])).numpy()
+    rq, rs = lib.quant_rows_pre(_bits(x)[rows], 1, tbits)
+    assert np.array_equal(xs.cpu().numpy().reshape(-1)[rows].view(np.uint32), rs.reshape(-1).view(np.uint32))
+    assert np.array_equal(xq.cpu().numpy()[rows], rq)
