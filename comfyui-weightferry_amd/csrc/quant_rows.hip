@@ -498,9 +498,19 @@ __global__ __launch_bounds__(256) void quant_convrot(const uint16_t* __restrict_
 // widest rows taken: 32768 values (one workgroup of four waves per row)
 constexpr int kMaxRowK = 32768;
 
+// Wide rows, many of them, are bound by memory, and more of them in flight than three workgroups a CU (two at the widest)
+// slow it: LDS that is asked for and not used keeps to that. us without and with it (MI355X): 16384 x 13824 124.7 and 115.4,
+// 4096 x 20480 42.7 and 39.8, 8192 x 32768 162.4 and 143.5; but 16384 x 8208 73.1 and 76.9, 1024 x 9216 6.7 and 7.1. (Before
+// the maxima went over 16-bit halves the registers kept to it: 122.3, 41.5, 156.6, 75.0, 7.3.)
+static size_t plain_lds(int64_t M, int K) {
+    if (M < 4096 || K < 9216) return 0;
+    return K <= 26624 ? 52 * 1024 : 63 * 1024;
+}
+
 template <int CPL, int W>
 static void launch_plain(const uint16_t* x, int64_t M, int K, int8_t* xq, float* xs, hipStream_t s) {
-    quant_plain<CPL, W><<<dim3((unsigned)((M + 4 / W - 1) / (4 / W))), 256, 0, s>>>(x, M, K, xq, xs);
+    const size_t lds = W == 1 ? 0 : plain_lds(M, K);
+    quant_plain<CPL, W><<<dim3((unsigned)((M + 4 / W - 1) / (4 / W))), 256, lds, s>>>(x, M, K, xq, xs);
 }
 
 static void launch_plain_rows(const uint16_t* x, int64_t M, int K, int8_t* xq, float* xs, hipStream_t s) {

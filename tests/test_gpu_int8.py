@@ -479,3 +479,14 @@ def test_gelu_table_in_lds_or_memory(native, M, K):
     rq, rs = lib.quant_rows_pre(_bits(x)[rows], 1, tbits)
     assert np.array_equal(xs.cpu().numpy().reshape(-1)[rows].view(np.uint32), rs.reshape(-1).view(np.uint32))
     assert np.array_equal(xq.cpu().numpy()[rows], rq)
+
+
+@pytest.mark.parametrize("M,K", [(4095, 9216), (4096, 9216), (4097, 26624), (4096, 26640)])
+def test_plain_rows_at_the_limits_of_their_launches(native, M, K):
+    # the widths and row counts where the number of workgroups a CU takes changes; the first and the last rows
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(K), dtype=torch.float32).to(torch.bfloat16)
+    xq, xs = gpu_quant(native, x.cuda(), 0)
+    rows = [0, 1, M // 2, M - 1]
+    rq, rs = lib.quant_rows(_bits(x[rows]), 0)
+    assert np.array_equal(xs.cpu().numpy().reshape(-1)[rows].view(np.uint32), rs.reshape(-1).view(np.uint32))
+    assert np.array_equal(xq.cpu().numpy()[rows], rq)
