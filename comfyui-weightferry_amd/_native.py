@@ -21,6 +21,13 @@ OK, EINVAL, EUNSUPPORTED, EHIP = 0, -1, -2, -3
 
 _p, _i64, _int, _sz = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_size_t
 
+
+class I8Plan(ctypes.Structure):
+    """wf_i8_plan: how an int8 product runs (wf_linear_i8_plan)."""
+    _fields_ = [("tile_rows", ctypes.c_int32), ("tile_columns", ctypes.c_int32), ("slices", ctypes.c_int32),
+                ("workspace_bytes", _i64), ("whole_ns", _i64)]
+
+
 # every symbol of include/weightferry.h: name -> (restype, argtypes)
 EXPORTS = {
     "wf_abi_version": (_int, []),
@@ -36,6 +43,7 @@ EXPORTS = {
     "wf_linear_i8_residual": (_int, [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p]),
     "wf_linear_i8_workspace": (_int, [_i64, _i64, _i64, ctypes.POINTER(_i64)]),
     "wf_linear_i8_ws": (_int, [_p, _p, _p, _p, _p, _p, _p, _p, _int, _i64, _i64, _i64, _i64, _p, _i64, _p]),
+    "wf_linear_i8_plan": (_int, [_i64, _i64, _i64, _i64, ctypes.POINTER(I8Plan)]),
     "wf_linear_gguf": (_int, [_p, _i64, _i64, _p, _i64, _int, _i64, _p, _p, _int, _p]),
     "wf_linear_gguf_workspace": (_int, [_i64, _i64, _i64, ctypes.POINTER(_i64)]),
     "wf_linear_gguf_ws": (_int, [_p, _i64, _i64, _p, _i64, _int, _i64, _p, _p, _int, _p, _i64, _p]),

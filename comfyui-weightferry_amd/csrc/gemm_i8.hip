@@ -600,20 +600,26 @@ static int64_t dl_cost(int M, int N, int bm, int bn, int64_t eff) {
     return (tiles + 255) / 256 * bm * bn * 1000 / eff;
 }
 
-template <int OUT>
-static void launch_dl(const int8_t* A, const int8_t* B, const float* xs, const float* ws, const void* bias,
-                      void* out, int M, int N, int K, Residual r, bool resid, hipStream_t s) {
+// columns of the 256-row tiling with the least modelled time, or 160: the 128 x 160 tiling
+static int dl_columns(int M, int N) {
     const int64_t c320 = dl_cost(M, N, 256, 320, 1030), c256 = dl_cost(M, N, 256, 256, 1000);
     const int64_t c128 = dl_cost(M, N, 256, 128, 780), c160 = dl_cost(M, N, 128, 160, 581);
     const int64_t best = std::min(std::min(c320, c256), std::min(c128, c160));
-    if (c160 == best && K % 128 == 0) launch_dl_shape<4, 1, 1, 5, OUT, 128>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
+    return c160 == best ? 160 : c128 == best ? 128 : c256 == best ? 256 : 320;
+}
+
+template <int OUT>
+static void launch_dl(const int8_t* A, const int8_t* B, const float* xs, const float* ws, const void* bias,
+                      void* out, int M, int N, int K, Residual r, bool resid, hipStream_t s) {
+    const int bn = dl_columns(M, N);
+    if (bn == 160 && K % 128 == 0) launch_dl_shape<4, 1, 1, 5, OUT, 128>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
     else if (K % 128 == 0) {
-        if (c128 == best) launch_wl_shape<2, 2, 4, 2, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
-        else if (c256 == best) launch_wl_shape<2, 4, 4, 2, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
+        if (bn == 128) launch_wl_shape<2, 2, 4, 2, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
+        else if (bn == 256) launch_wl_shape<2, 4, 4, 2, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
         else launch_wl_shape<4, 2, 2, 5, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
-    } else if (c160 == best) launch_dl_shape<4, 1, 1, 5, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
-    else if (c128 == best) launch_dl_shape<2, 2, 4, 2, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
-    else if (c256 == best) launch_dl_shape<2, 4, 4, 2, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
+    } else if (bn == 160) launch_dl_shape<4, 1, 1, 5, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
+    else if (bn == 128) launch_dl_shape<2, 2, 4, 2, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
+    else if (bn == 256) launch_dl_shape<2, 4, 4, 2, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
     else launch_dl_shape<4, 2, 2, 5, OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s);
 }
 
@@ -622,23 +628,19 @@ struct I8Form {
     int bm, bn;          // tile
     int stage, turn;     // ns of a 128-byte stage: alone on a CU; its share of the CU when a CU has several workgroups
 };
-// Times fitted on MI355X to 1,900 measurements (rows 4-5152, 1024 <= N, K <= 13824, weights out of the last-level
-// cache); over them the choice is 1.40 times as fast as the 256-row and 128 x 160 tilings alone and within 3 % of the
-// best form measured, and one shape in 130 is over 1 % slower than before (1536 x 2048 x 8192, 4 %). Against the tilings
-// alone (us): 5120 x 5120 at 16 / 64 / 128 / 256 / 512 rows 13.3 / 15.2 / 17.5 / 23.3 / 32.7 against 27.9 / 29.6 / 33.7
-// / 33.0 / 32.7; 5120 x 13824 at 16 / 256 / 768 rows 23.8 / 38.9 / 70.5 against 66.4 / 76.2 / 78.2; 2048 x 8192 at 256
-// rows 17.4 against 44.7; 1024 x 1024 at 64 rows 4.7 against 9.0.
+// Times fitted on MI355X to 1,900 measurements (rows 4-5152, 1024 <= N, K <= 13824, weights out of the last-level cache).
 constexpr I8Form kI8Forms[] = {{32, 128, 705, 394},    {64, 128, 806, 460},    {128, 128, 900, 562},
                                {256, 192, 1334, 1276}, {256, 256, 1481, 1486}, {256, 320, 1667, 1608}};
 // ns of a 256 x 256 tile's epilogue; of the sums' launch; bytes per ns of the slices' way through memory and of a
 // weight's, which also costs kI8Start
 constexpr int64_t kI8Epilogue = 2992, kI8Sum = 4523, kI8SumBytes = 6804, kI8Stream = 4854, kI8Start = 3000;
-constexpr int kI8Ring = 6;                      // gemm_i8_dl's 128 x 160 tiles, 4-stage ring
+constexpr int kI8Tiles = 6;                     // launch_dl's tiling, whichever that is
 constexpr int kI8MinStages = 3, kI8MaxSlices = 16;
 
 struct I8Plan {
     int form, slices, per;
     int64_t part_bytes;
+    int64_t whole_ns;    // modelled time without slices
 };
 
 static int64_t tiles_of(int64_t M, int64_t N, int bm, int bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); }
@@ -656,25 +658,61 @@ static int64_t i8_ring_time(int64_t tiles, int64_t nk) { return 4000 + (tiles + 
 
 static bool i8_modelled(int64_t M, int64_t N, int64_t K) { return K % 128 == 0 && tiles_of(M, N, 256, 320) < 256; }
 
+// 256 x 128 tiles (launch_dl's, with four waves); a low estimate
+static int64_t i8_narrow_time(int64_t tiles, int64_t nk) { return 5000 + (tiles + 255) / 256 * nk * 1150; }
+
+// The model's best form replaces launch_dl's tiling only where that measured faster both with the weight in the
+// last-level cache and with it outside (770 random shapes of 3-6000 rows: 1.17 times as fast on average, none more than
+// 1.1 % slower). It stays away from
+//  * 32-row tiles where they take more than one turn or the weight is over 24 MB: two stages in flight wait for memory
+//    where the ring has four (8800 x 2560 at 128 rows 17.8 against 15.1 us, 7744 x 7168 at 6 rows 44 against 38);
+//  * K < 2048, where epilogues outweigh the modelled loop, unless it is 10 % ahead of the ring (2138 x 1152 at 2718 rows
+//    21.7 against 19.4; 11464 x 1280 at 219 rows 12.0 against 11.1);
+//  * two turns of 128 x 128 tiles against 256-row tiles (8544 x 7680 at 746 rows 70.9 against 60.2), unless they are 10 %
+//    ahead of 256 x 128.
+static int i8_whole_form(int64_t M, int64_t N, int64_t K, int bn, int64_t* ns) {
+    const int64_t nk = K / 128, ring = i8_ring_time(tiles_of(M, N, 128, 160), nk);
+    const int64_t narrow = bn == 128 ? i8_narrow_time(tiles_of(M, N, 256, 128), nk) : INT64_MAX / 16;
+    int form = kI8Tiles;
+    int64_t t = INT64_MAX, tiles = 0;
+    for (int f = 0; f < kI8Tiles; f++) {
+        const int64_t n = tiles_of(M, N, kI8Forms[f].bm, kI8Forms[f].bn), v = i8_time(kI8Forms[f], n, 1, nk, N * K);
+        if (v < t) { t = v; form = f; tiles = n; }
+    }
+    *ns = std::min(std::min(t, ring), narrow);
+    if (form == 0 && (tiles > 256 || N * K > 24000000)) return kI8Tiles;
+    if (K < 2048) return bn == 160 && 10 * t <= 9 * ring ? form : kI8Tiles;
+    if (form == 2 && bn != 160 && tiles > 256) return bn == 128 && 10 * t <= 9 * narrow ? form : kI8Tiles;
+    return t <= ring ? form : kI8Tiles;
+}
+
+// Slices stay within one turn of workgroups and need 15 % of modelled time; against 256 x 128 tiles, which the model knows
+// less well, 25 % (13264 x 12928 at 434 rows: 97.7 in slices against 85.3 us). Over the same shapes 1.48 times as fast as
+// launch_dl's tilings, none more than 1.1 % slower; weights out of the cache (us, GPU time): 5120 x 5120 at 16 / 64 / 256
+// rows 13.3 / 15.2 / 23.3 against 27.9 / 29.6 / 33.0, 2048 x 8192 at 256 rows 17.4 against 44.7, 5120 x 13824 at 1560 rows
+// 125 against 152. (What the second launch costs a caller's thread is the caller's to weigh: whole_ns.)
 static I8Plan i8_plan(int64_t M, int64_t N, int64_t K, int64_t max_part) {
     const int64_t nk = K / 128;
-    I8Plan best{kI8Ring, 1, (int)nk, 0};
-    int64_t t = INT64_MAX;
-    for (int f = 0; f < 6; f++) {
+    const int bn = dl_columns((int)M, (int)N);
+    I8Plan best{kI8Tiles, 1, (int)nk, 0, 0};
+    best.form = i8_whole_form(M, N, K, bn, &best.whole_ns);
+    if (max_part <= 0) return best;
+    int64_t t = best.whole_ns * (bn == 128 ? 75 : 85) / 100;
+    for (int f = 0; f < kI8Tiles; f++) {
         const I8Form& F = kI8Forms[f];
         const int64_t tiles = tiles_of(M, N, F.bm, F.bn);
-        int64_t last = 0;
-        for (int s = 1; s <= kI8MaxSlices; s++) {
+        int64_t last = 1;
+        for (int s = 2; s <= kI8MaxSlices; s++) {
             const int64_t per = (nk + s - 1) / s, slices = (nk + per - 1) / per;
-            if (s > 1 && (per < kI8MinStages || slices == last || tiles * slices > 1024)) continue;
+            if (per < kI8MinStages) break;
+            if (slices == last || tiles * slices > 256) continue;
             last = slices;
-            const int64_t part = slices > 1 ? tiles * slices * F.bm * F.bn * 4 : 0;
+            const int64_t part = tiles * slices * F.bm * F.bn * 4;
             if (part > std::min(max_part, kI8MaxPart)) continue;
             const int64_t v = i8_time(F, tiles, slices, per, N * K);
-            if (v < t) { t = v; best = {f, (int)slices, (int)per, part}; }
+            if (v < t) { t = v; best.form = f; best.slices = (int)slices; best.per = (int)per; best.part_bytes = part; }
         }
     }
-    if (i8_ring_time(tiles_of(M, N, 128, 160), nk) < t) best = {kI8Ring, 1, (int)nk, 0};
     return best;
 }
 
@@ -707,7 +745,7 @@ static void launch_i8_plan(const I8Plan& p, const int8_t* A, const int8_t* B, co
     case 3: launch_i8_form<4, 2, 2, 3, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
     case 4: launch_i8_form<2, 4, 4, 2, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
     case 5: launch_i8_form<4, 2, 2, 5, OUT>(p, A, B, xs, ws, bias, out, M, N, K, r, resid, part, s); break;
-    default: launch_dl_shape<4, 1, 1, 5, OUT, 128>(A, B, xs, ws, bias, out, M, N, K, r, resid, s); break;
+    default: launch_dl<OUT>(A, B, xs, ws, bias, out, M, N, K, r, resid, s); break;
     }
 }
 
@@ -828,6 +866,34 @@ extern "C" int wf_linear_i8_workspace(int64_t M, int64_t N, int64_t K, int64_t* 
     if (M < 0 || N < 0 || K <= 0) { set_error("wf_linear_i8_workspace: M, N, K"); return WF_EINVAL; }
     if (M > 0 && N > 0 && M < (1LL << 31) && N < (1LL << 31) && K <= 131071 && i8_modelled(M, N, K))
         *bytes = i8_plan(M, N, K, INT64_MAX).part_bytes;
+    return WF_OK;
+}
+
+extern "C" int wf_linear_i8_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, wf_i8_plan* plan) {
+    using namespace wf;
+    if (!plan) { set_error("wf_linear_i8_plan: null out-pointer"); return WF_EINVAL; }
+    *plan = {};
+    if (M <= 0 || N <= 0 || K <= 0) { set_error("wf_linear_i8_plan: M, N, K"); return WF_EINVAL; }
+    if (M >= (1LL << 31) || N >= (1LL << 31) || K > 131071 || K % 16) {
+        set_error("wf_linear_i8_plan: a product the kernels do not take");
+        return WF_EUNSUPPORTED;
+    }
+    plan->slices = 1;
+    int form = kI8Tiles;
+    if (i8_modelled(M, N, K)) {
+        const I8Plan p = i8_plan(M, N, K, workspace_bytes);
+        form = p.form;
+        plan->slices = p.slices;
+        plan->workspace_bytes = p.part_bytes;
+        plan->whole_ns = p.whole_ns;
+    }
+    if (form != kI8Tiles) {
+        plan->tile_rows = kI8Forms[form].bm;
+        plan->tile_columns = kI8Forms[form].bn;
+    } else if (K % kDlBK == 0) {
+        plan->tile_columns = dl_columns((int)M, (int)N);
+        plan->tile_rows = plan->tile_columns == 160 ? 128 : 256;
+    }
     return WF_OK;
 }
 

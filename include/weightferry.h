@@ -110,6 +110,15 @@ int wf_linear_i8_ws(const int8_t* xq, const int8_t* wq, const float* xs, const f
                     const void* gate_bf16, const void* resid_bf16, void* out, int out_dt, int64_t M, int64_t N,
                     int64_t K, int64_t rows_per_group, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* How a product runs when it may use a workspace of workspace_bytes (0: wf_linear_i8, wf_linear_i8_residual; INT64_MAX:
+ * wf_linear_i8_ws). tile_rows 0: the kernel for K that is not a multiple of 64. whole_ns is the modelled GPU time without
+ * slices, 0 where nothing is modelled (then there are no slices): a caller bound by its own thread can do without them. */
+typedef struct {
+    int32_t tile_rows, tile_columns, slices;
+    int64_t workspace_bytes, whole_ns;
+} wf_i8_plan;
+int wf_linear_i8_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, wf_i8_plan* plan);
+
 /* ------------------------------------------------------------------------------- fused dequant + bf16 GEMM
  * y[m, n] = bf16(sum_k x[m, k] * W[n, k] (+ bias[n])) with W given as GGUF K-quant blocks (qtype 12 Q4_K, 13 Q5_K, 14
  * Q6_K; [N, K] row-major in 256-value super-blocks, wq_bytes = N * K / 256 * block bytes; also qtype 8 Q8_0, 34 bytes

@@ -490,3 +490,53 @@ def test_plain_rows_at_the_limits_of_their_launches(native, M, K):
     rq, rs = lib.quant_rows(_bits(x[rows]), 0)
     assert np.array_equal(xs.cpu().numpy().reshape(-1)[rows].view(np.uint32), rs.reshape(-1).view(np.uint32))
     assert np.array_equal(xq.cpu().numpy()[rows], rq)
+
+
+def _plan(native, M, N, K, workspace):
+    p = native.I8Plan()
+    assert native.lib().wf_linear_i8_plan(M, N, K, workspace, ctypes.byref(p)) == 0, native.last_error()
+    return p
+
+
+# every tiling wf_linear_i8 and wf_linear_i8_ws choose by the model, with a partial last tile in rows and columns, odd and
+# whole-run widths, two gate groups that meet inside a tile
+@pytest.mark.parametrize("tile,sliced,M,N,K", [
+    ((32, 128), False, 2, 266, 128), ((64, 128), False, 162, 11271, 384), ((128, 128), False, 1670, 3001, 2048),
+    ((256, 192), False, 1182, 6982, 2048), ((256, 256), False, 3002, 3001, 384), ((256, 128), False, 2002, 4008, 640),
+    ((256, 320), False, 4002, 4993, 384), ((128, 160), False, 1002, 5001, 640), ((128, 160), False, 1022, 4999, 128),
+    ((32, 128), True, 34, 2040, 8192), ((64, 128), True, 302, 1287, 5120), ((128, 128), True, 130, 2047, 8192),
+    ((256, 192), True, 134, 5566, 6400), ((256, 256), True, 1142, 1002, 11520), ((256, 320), True, 3190, 619, 12928)])
+def test_every_planned_tiling(native, tile, sliced, M, N, K):
+    plan = _plan(native, M, N, K, 1 << 62 if sliced else 0)
+    assert (plan.tile_rows, plan.tile_columns) == tile and (plan.slices > 1) == sliced, \
+        (plan.tile_rows, plan.tile_columns, plan.slices)
+    g = torch.Generator().manual_seed(M + N)
+    xq, wq = _rand_i8(g, (M, K)), _rand_i8(g, (N, K))
+    xs, ws = torch.rand(M, generator=g) * 0.05 + 1e-3, torch.rand(N, generator=g) * 0.002 + 1e-5
+    bias, resid = (torch.randn(s, generator=g).to(torch.bfloat16) for s in ((N,), (M, N)))
+    gate = torch.randn((2, N), generator=g).to(torch.bfloat16)
+    part = torch.full((max(1, plan.workspace_bytes),), 0x5A, dtype=torch.uint8, device="cuda")
+    d = {k: v.cuda() for k, v in dict(xq=xq, wq=wq, xs=xs, ws=ws, bias=bias, gate=gate, resid=resid).items()}
+    # the sum exact in the float64 product (|acc| < 2^28), then one rounding to float32 as the kernel's
+    t = ((d["xq"].double() @ d["wq"].double().T).float() * d["xs"][:, None]) * d["ws"][None, :]
+    stream = native.stream_of(part.device)
+    for residual in (False, True):
+        y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+        ops = [d[k].data_ptr() for k in ("xq", "wq", "xs", "ws")]
+        if sliced:
+            p = [None if residual else d["bias"].data_ptr(), d["gate"].data_ptr() if residual else None,
+                 d["resid"].data_ptr() if residual else None]
+            rc = native.lib().wf_linear_i8_ws(*ops, *p, y.data_ptr(), 1, M, N, K, M // 2, part.data_ptr(), part.numel(),
+                                              stream)
+        elif residual:
+            rc = native.lib().wf_linear_i8_residual(*ops, d["gate"].data_ptr(), d["resid"].data_ptr(), y.data_ptr(), M, N,
+                                                    K, M // 2, stream)
+        else:
+            rc = native.lib().wf_linear_i8(*ops, d["bias"].data_ptr(), y.data_ptr(), 1, M, N, K, stream)
+        assert rc == 0, native.last_error()
+        if residual:
+            ref = torch.addcmul(d["resid"], d["gate"].repeat_interleave(M // 2, 0), t.to(torch.bfloat16))
+        else:
+            ref = (t + d["bias"].float()).to(torch.bfloat16)
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), ref.view(torch.int16)), residual

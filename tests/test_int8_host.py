@@ -2,6 +2,9 @@
 and the shared-quantisation cache (enhancers/fused_int8.py:311-332 of the reference); _int8_quantised declines
 every case outside the reference's eligibility (:129-147), and _shared_forward then runs
 torch.nn.functional.linear and counts the fallback (:279-292); a pending input is materialised for the fallback."""
+import ctypes
+
+import pytest
 import torch
 
 from conftest import sub
@@ -9,6 +12,7 @@ from fake_quant import FakeQT, Lin
 
 fi = sub("enhancers.fused_int8")
 fs = sub("enhancers.fused_state")
+native = sub("_native")
 
 
 def _weight(n=16, k=256, **kw):
@@ -85,3 +89,48 @@ def test_residual_forward_without_pending_residual_is_shared_forward():
 def test_int8_linear_declines_cpu():
     assert fi.int8_linear(torch.randn(4, 256).to(torch.bfloat16), torch.zeros(8, 256, dtype=torch.int8),
                           torch.ones(8)) is None
+
+
+def _plan(M, N, K, workspace=1 << 62):
+    p = native.I8Plan()
+    rc = native.lib().wf_linear_i8_plan(M, N, K, workspace, ctypes.byref(p))
+    return rc, p
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    # the shapes whose modelled tiling measured slower than the one they had
+    (600, 13824, 5120, (256, 256)), (135, 8256, 1920, (128, 160)), (197, 6975, 2560, (128, 160)),
+    (6, 7744, 7168, (128, 160)), (25, 12560, 6144, (128, 160)), (303, 4848, 2176, (128, 160)),
+    (700, 8048, 11264, (256, 128)), (746, 8544, 7680, (256, 128)), (867, 8288, 5888, (256, 256)),
+    (219, 11464, 1280, (128, 160)), (2718, 2138, 1152, (256, 128)), (434, 13264, 12928, (256, 128)),
+    # those the tests of the tilings name
+    (4000, 5000, 512, (256, 320)), (3000, 3000, 384, (256, 256)), (2000, 4000, 640, (256, 128)),
+    (1024, 5000, 512, (128, 160)), (1024, 4992, 128, (128, 160))])
+def test_plan_keeps_the_tilings_that_measured_faster(M, N, K, tile):
+    for workspace in (0, 1 << 62):
+        rc, p = _plan(M, N, K, workspace)
+        if p.slices == 1:
+            assert rc == 0 and (p.tile_rows, p.tile_columns) == tile and p.workspace_bytes == 0
+
+
+@pytest.mark.parametrize("M,N,K", [(746, 2592, 4608), (746, 8544, 7680), (434, 13264, 12928), (4748, 1404, 11776),
+                                   (1275, 5949, 9728), (679, 1888, 3328), (2826, 1936, 9984), (1094, 1464, 6272)])
+def test_plan_leaves_out_slices_that_measured_slower(M, N, K):
+    rc, p = _plan(M, N, K)
+    assert rc == 0 and p.slices == 1 and p.workspace_bytes == 0
+
+
+def test_plan_query():
+    need = ctypes.c_int64()
+    for M, N, K in ((256, 5120, 5120), (1560, 5120, 13824), (16, 5120, 5120)):
+        rc, p = _plan(M, N, K)
+        assert rc == 0 and p.slices > 1 and p.whole_ns > 20000
+        assert native.lib().wf_linear_i8_workspace(M, N, K, ctypes.byref(need)) == 0 and need.value == p.workspace_bytes
+        rc, q = _plan(M, N, K, p.workspace_bytes - 1)            # fewer slices, or none
+        assert rc == 0 and q.workspace_bytes < p.workspace_bytes
+        assert _plan(M, N, K, 0)[1].slices == 1
+    rc, p = _plan(300, 1000, 208)                                # the kernel for K % 64 != 0
+    assert rc == 0 and p.tile_rows == 0 and p.slices == 1 and p.whole_ns == 0
+    assert _plan(0, 8, 128)[0] == native.EINVAL and _plan(8, 8, 0)[0] == native.EINVAL
+    assert _plan(8, 8, 131088)[0] == native.EUNSUPPORTED and _plan(8, 8, 24)[0] == native.EUNSUPPORTED
+    assert native.lib().wf_linear_i8_plan(8, 8, 128, 0, None) == native.EINVAL
