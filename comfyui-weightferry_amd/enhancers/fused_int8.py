@@ -15,7 +15,7 @@ What a call here computes, for a bf16 input x [m, k] and an int8 ConvRot weight 
   (``mod``), LayerNorm then scale-and-shift (``lnmod``), or GELU (``gelu``) -- and the layer receives ``marker``;
   the operation then runs inside the quantiser and the real input is never written;
 * the int8 GEMM with the scale epilogue, or with the gated residual ``x_res + gate * out`` when the block left its
-  residual pending (``wf_linear_i8_ws``).
+  residual pending (``wf_linear_i8``, ``wf_linear_i8_residual``, or ``wf_linear_i8_ws`` in K slices).
 
 The per-thread state lives in ``fused_state._tls``: ``qkv`` (the shared quantisation, a dict while ``_Overrides``
 is active), ``pre`` (the pending input), ``res`` (the pending residual). The names of this module's functions and
@@ -59,46 +59,69 @@ def quantise_rows(x_2d, mode):
     return (x_q, x_s) if _native.check(rc, "wf_quant_rows_i8") else None
 
 
-_needs = {}                  # (m, n, k) -> the bytes wf_linear_i8_workspace gives
+# K slices (wf_linear_i8_ws) save GPU time and cost this thread a second launch and a workspace, about 5 us. A product that
+# takes less GPU time than its call takes the thread gains nothing and is that much slower, so it runs whole: below
+# _LEAST_NS for int8_linear (its call 24 us whole, 29 in slices on MI355X: 2048 x 2048 at 4-150 rows 24.2 against 29.4 us,
+# 5120 x 5120 at 16 rows 32.6 against 29.2), below _BLOCK_LEAST_NS for a layer of a block, whose eligibility checks take
+# longer (a QKV of three layers 315 us whole, 331 in slices at 2048 and 4096 wide, 32-256 rows).
+_LEAST_NS, _BLOCK_LEAST_NS = 26_000, 100_000
+_plans = {}                  # (m, n, k) -> (the bytes K slices need, 0: none; the modelled ns without them)
 
 
-def _workspace(m, n, k, dev):
-    """The workspace of an int8 GEMM of this shape (K-slice sums), or None where it needs none. A new tensor each call:
-    torch's allocator hands its memory on only to work queued later on this stream."""
-    need = _needs.get((m, n, k))
-    if need is None:
-        v = ctypes.c_int64()
-        _native.call("wf_linear_i8_workspace", m, n, k, ctypes.byref(v))
-        if len(_needs) > 4096:
-            _needs.clear()
-        need = _needs[m, n, k] = v.value
-    return torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+def _plan(m, n, k):
+    """_plans' entry for a shape, asked of the library once (the answer depends on the shape only)."""
+    p = _native.I8Plan()
+    rc = _native.lib().wf_linear_i8_plan(m, n, k, 1 << 62, ctypes.byref(p))
+    if len(_plans) > 4096:
+        _plans.clear()
+    plan = _plans[m, n, k] = (0, 0) if rc else (p.workspace_bytes, p.whole_ns)
+    return plan
 
 
-def _linear_i8(x_q, x_s, w_q, ws, bias, gate, resid, out, rows_per_gate):
-    """wf_linear_i8_ws; False when the library declines."""
+def _workspace(nbytes, dev):
+    """Device memory for K slices. A new tensor each call: torch's allocator hands its memory on only to work queued
+    later on this stream."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+
+
+def _linear_i8(x_q, x_s, w_q, ws, bias, gate, resid, out, rows_per_gate, least_ns):
+    """One int8 product, plain or (gate, resid) residual; False when the library declines."""
     m, k = x_q.shape
     n, dev = w_q.shape[0], x_q.device
+    lib = _native.lib()
     with _native.on_device(dev):
-        part = _workspace(m, n, k, dev)
-        rc = _native.lib().wf_linear_i8_ws(
-            x_q.data_ptr(), w_q.data_ptr(), x_s.data_ptr(), ws.data_ptr(), None if bias is None else bias.data_ptr(),
-            None if gate is None else gate.data_ptr(), None if resid is None else resid.data_ptr(), out.data_ptr(),
-            1 if out.dtype == torch.bfloat16 else 0, m, n, k, rows_per_gate, None if part is None else part.data_ptr(),
-            0 if part is None else part.numel(), _stream(dev))
-    return _native.check(rc, "wf_linear_i8")
+        stream, code = _stream(dev), 1 if out.dtype == torch.bfloat16 else 0
+        bias_ptr = None if bias is None else bias.data_ptr()
+        need, whole_ns = _plans.get((m, n, k)) or _plan(m, n, k)
+        part = _workspace(need, dev) if need and whole_ns >= least_ns else None
+        if part is not None:
+            what = "wf_linear_i8_ws"
+            rc = lib.wf_linear_i8_ws(x_q.data_ptr(), w_q.data_ptr(), x_s.data_ptr(), ws.data_ptr(), bias_ptr,
+                                     None if gate is None else gate.data_ptr(),
+                                     None if resid is None else resid.data_ptr(), out.data_ptr(), code, m, n, k,
+                                     rows_per_gate, part.data_ptr(), need, stream)
+        elif gate is None:
+            what = "wf_linear_i8"
+            rc = lib.wf_linear_i8(x_q.data_ptr(), w_q.data_ptr(), x_s.data_ptr(), ws.data_ptr(), bias_ptr,
+                                  out.data_ptr(), code, m, n, k, stream)
+        else:
+            what = "wf_linear_i8_residual"
+            rc = lib.wf_linear_i8_residual(x_q.data_ptr(), w_q.data_ptr(), x_s.data_ptr(), ws.data_ptr(),
+                                           gate.data_ptr(), resid.data_ptr(), out.data_ptr(), m, n, k, rows_per_gate,
+                                           stream)
+    return _native.check(rc, what)
 
 
-def gemm(x_q, x_s, w_q, ws, out_dtype=torch.bfloat16, bias=None):
+def gemm(x_q, x_s, w_q, ws, out_dtype=torch.bfloat16, bias=None, least_ns=_LEAST_NS):
     """out[m, n] = out_dtype((float(sum_k x_q[m, k] w_q[n, k]) * x_s[m]) * ws[n] (+ bias[n])), the sum exact in
-    int32; None when the library declines."""
+    int32; None when the library declines. In K slices only where the product takes ``least_ns`` or more without."""
     out = torch.empty((x_q.shape[0], w_q.shape[0]), dtype=out_dtype, device=x_q.device)
-    return out if _linear_i8(x_q, x_s, w_q, ws, bias, None, None, out, 1) else None
+    return out if _linear_i8(x_q, x_s, w_q, ws, bias, None, None, out, 1, least_ns) else None
 
 
 def _gemm_residual(q, gate_2d, resid_2d, out_2d, rows_per_gate):
     """The residual form: out = bf16(resid + gate[row // rows_per_gate] * linear) over q's rows."""
-    return _linear_i8(q.x_q, q.x_s, q.w_q, q.ws, None, gate_2d, resid_2d, out_2d, rows_per_gate)
+    return _linear_i8(q.x_q, q.x_s, q.w_q, q.ws, None, gate_2d, resid_2d, out_2d, rows_per_gate, _BLOCK_LEAST_NS)
 
 
 # ------------------------------------------------------------------------------------- a direct entry point
@@ -375,7 +398,7 @@ def _int8_linear_shared(x, weight, bias):
     q = _int8_quantised(x, weight, bias)
     if q is None:
         return None
-    out = gemm(q.x_q, q.x_s, q.w_q, q.ws, q.dtype)
+    out = gemm(q.x_q, q.x_s, q.w_q, q.ws, q.dtype, least_ns=_BLOCK_LEAST_NS)
     if out is None or x.dim() == 2:
         return out
     return out.reshape(*x.shape[:-1], q.n)

@@ -134,3 +134,50 @@ def test_plan_query():
     assert _plan(0, 8, 128)[0] == native.EINVAL and _plan(8, 8, 0)[0] == native.EINVAL
     assert _plan(8, 8, 131088)[0] == native.EUNSUPPORTED and _plan(8, 8, 24)[0] == native.EUNSUPPORTED
     assert native.lib().wf_linear_i8_plan(8, 8, 128, 0, None) == native.EINVAL
+
+
+class _Calls:
+    """The native library with its int8 products recorded instead of run."""
+
+    def __init__(self):
+        self.names, self.real = [], native.lib()
+
+    def __getattr__(self, name):
+        if name not in ("wf_linear_i8", "wf_linear_i8_residual", "wf_linear_i8_ws"):
+            return getattr(self.real, name)
+        return lambda *a: self.names.append(name) or self.rc
+
+    rc = 0
+
+
+def _products(monkeypatch, calls, m, n, k, least_ns, residual=False):
+    """The entry points one product goes through."""
+    monkeypatch.setattr(native, "lib", lambda: calls)
+    monkeypatch.setattr(fi, "_stream", lambda dev: None)
+    x_q, w_q = torch.empty((m, k), dtype=torch.int8), torch.empty((n, k), dtype=torch.int8)
+    x_s, ws = torch.empty((m, 1)), torch.empty(n)
+    out = torch.empty((m, n), dtype=torch.bfloat16)
+    gate = out[:1] if residual else None
+    assert fi._linear_i8(x_q, x_s, w_q, ws, None, gate, out if residual else None, out, m, least_ns)
+    return calls.names
+
+
+@pytest.mark.parametrize("m,n,k,direct,block", [
+    (64, 2048, 2048, False, False), (150, 2048, 2048, False, False), (64, 1111, 4096, False, False),   # shorter than a call
+    (16, 5120, 5120, True, False), (256, 5120, 5120, True, False), (300, 2048, 8192, True, False),
+    (16, 5120, 13824, True, False),                                                  # longer than int8_linear's call
+    (1560, 5120, 13824, True, True), (5152, 2048, 8192, False, False)])              # longer than a block's layer
+def test_slices_only_where_the_call_is_longer_than_its_host_time(monkeypatch, m, n, k, direct, block):
+    assert _products(monkeypatch, _Calls(), m, n, k, fi._LEAST_NS) == ["wf_linear_i8_ws" if direct else "wf_linear_i8"]
+    assert _products(monkeypatch, _Calls(), m, n, k, fi._BLOCK_LEAST_NS) == ["wf_linear_i8_ws" if block else "wf_linear_i8"]
+    assert _products(monkeypatch, _Calls(), m, n, k, fi._BLOCK_LEAST_NS, residual=True) == [
+        "wf_linear_i8_ws" if block else "wf_linear_i8_residual"]
+
+
+def test_failures_name_the_entry_point_that_ran(monkeypatch):
+    calls = _Calls()
+    calls.rc = native.EINVAL
+    for m, n, k, residual, name in ((8, 64, 256, False, "wf_linear_i8"), (8, 64, 256, True, "wf_linear_i8_residual"),
+                                    (16, 5120, 5120, False, "wf_linear_i8_ws")):
+        with pytest.raises(native.NativeError, match=name + " failed"):
+            _products(monkeypatch, calls, m, n, k, 0, residual)
