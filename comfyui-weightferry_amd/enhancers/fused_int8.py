@@ -79,9 +79,12 @@ def _plan(m, n, k):
 
 
 def _workspace(nbytes, dev):
-    """Device memory for K slices. A new tensor each call: torch's allocator hands its memory on only to work queued
-    later on this stream."""
-    return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    """Device memory for K slices, or None when there is none left: the product runs whole then, with the same bits. A
+    new tensor each call: torch's allocator hands its memory on only to work queued later on this stream."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def _linear_i8(x_q, x_s, w_q, ws, bias, gate, resid, out, rows_per_gate, least_ns):

@@ -181,3 +181,21 @@ def test_failures_name_the_entry_point_that_ran(monkeypatch):
                                     (16, 5120, 5120, False, "wf_linear_i8_ws")):
         with pytest.raises(native.NativeError, match=name + " failed"):
             _products(monkeypatch, calls, m, n, k, 0, residual)
+
+
+def test_no_memory_for_slices_runs_the_product_whole(monkeypatch):
+    real, asked = torch.empty, []
+
+    def empty(*shape, **kw):
+        if kw.get("dtype") == torch.uint8:
+            asked.append(shape)
+            raise torch.OutOfMemoryError("no memory")
+        return real(*shape, **kw)
+    x = [real((16, 13824), dtype=torch.int8), real((16, 1)), real((5120, 13824), dtype=torch.int8), real(5120)]
+    calls = _Calls()
+    monkeypatch.setattr(native, "lib", lambda: calls)
+    monkeypatch.setattr(fi, "_stream", lambda dev: None)
+    monkeypatch.setattr(torch, "empty", empty)
+    assert fi.gemm(*x) is not None and calls.names == ["wf_linear_i8"] and len(asked) == 1
+    out = real((16, 5120), dtype=torch.bfloat16)
+    assert fi._linear_i8(*x, None, out[:1], out, out, 16, 0) and calls.names[1:] == ["wf_linear_i8_residual"]
