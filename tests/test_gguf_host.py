@@ -182,3 +182,30 @@ def test_comfy_memory_calls_release_pinned_copies(gd, monkeypatch):
     mm.soft_empty_cache(True)
     mm.unload_all_models()
     assert emptied == [1] and [c[0] for c in calls] == ["free_memory", "soft_empty_cache", "unload_all_models"]
+
+
+class _LoraCalls:
+    """The native library with its LoRA launches recorded instead of run."""
+
+    def __init__(self):
+        self.names = []
+
+    def __getattr__(self, name):
+        return lambda *a: self.names.append(name) or 0
+
+
+@pytest.mark.parametrize("up,down,rank,kernel", [
+    (torch.bfloat16, torch.bfloat16, 192, True), (torch.float16, torch.float16, 128, True),
+    (torch.bfloat16, torch.float32, 192, True), (torch.bfloat16, torch.bfloat16, 130, False),
+    (torch.float16, torch.bfloat16, 127, True), (torch.bfloat16, torch.bfloat16, 256, False),
+    (torch.float32, torch.float32, 64, True), (torch.float32, torch.float32, 80, False),
+    (torch.float32, torch.bfloat16, 96, True), (torch.float32, torch.bfloat16, 128, False),
+    (torch.float64, torch.bfloat16, 8, False), (torch.bfloat16, torch.bfloat16, 0, False)])
+def test_lora_route_by_rank_and_dtype(gd, monkeypatch, up, down, rank, kernel):
+    calls = _LoraCalls()
+    monkeypatch.setattr(gd._native, "lib", lambda: calls)
+    res = torch.zeros((24, 32), dtype=torch.bfloat16)
+    args = ((None, 0, 0, 0), torch.zeros((24, rank), dtype=up), torch.zeros((rank, 32), dtype=down), 1.0, res, "0", None)
+    assert gd._add_in_kernel(*args) is kernel
+    assert gd._add_in_kernel(*args) or gd._add_difference(*args)
+    assert calls.names == (["wf_dequant_lora"] * 2 if kernel else ["wf_dequant_add"])

@@ -195,3 +195,51 @@ def test_inference_mode_factors_use_the_kernel(native, fake_gguf):
             assert ok, where
     finally:
         gd.uninstall()
+
+
+def _integer_loras(shapes, n_out, n_in, dtypes):
+    """LoRAs whose factors are small integers: every float32 sum is exact, so the result is one set of bits."""
+    g = torch.Generator().manual_seed(sum(shapes))
+    return [(torch.randint(-8, 9, (n_out, r), generator=g).to(d), torch.randint(-8, 9, (r, n_in), generator=g).to(d), s)
+            for r, d, s in zip(shapes, dtypes, (0.0078125, -0.00390625))]
+
+
+@pytest.mark.parametrize("ranks,dtypes", [
+    ((256,), (torch.bfloat16,)), ((130,), (torch.float16,)), ((80,), (torch.float32,)), ((8,), (torch.float64,)),
+    ((16, 256), (torch.bfloat16, torch.bfloat16)), ((256, 16), (torch.float32, torch.bfloat16)),
+    ((200, 96), (torch.bfloat16, torch.float32))])
+def test_loras_beside_the_kernel(native, monkeypatch, ranks, dtypes):
+    # LoRAs that take torch.mm's difference (high ranks, float64), alone and before or after one that the kernel computes
+    gd = sub("enhancers.gguf_dequant")
+    n_out, n_in = 96, 512
+    raw = encode.random_blocks(13, n_out * n_in // 256, seed=5, family="normal")
+    loras = _integer_loras(ranks, n_out, n_in, dtypes)
+    routes, plain = [], gd._add_difference
+    monkeypatch.setattr(gd, "_add_difference", lambda *a: routes.append(a[1].shape[1]) or plain(*a))
+    for out, D in ((torch.bfloat16, BF16), (torch.float32, F32)):
+        del routes[:]
+        y = gd.dequantize_lora(torch.from_numpy(raw).cuda(), 13, (n_out, n_in), None, out, loras)
+        assert routes == [r for r in ranks if r != 16]
+        torch.cuda.synchronize()
+        ok, where = _same(_bits(y, D), _expected(raw, 13, F16, D, n_out, n_in, loras), D)
+        assert ok, where
+
+
+def test_lora_factor_the_kernel_declines(native):
+    # a device factor that starts at an odd value: not aligned to a pair of values, so the kernel declines it
+    gd = sub("enhancers.gguf_dequant")
+    n_out, n_in = 64, 256
+    raw = encode.random_blocks(8, n_out * n_in // 32, seed=6, family="normal")
+    (up, down, s), = _integer_loras((16,), n_out, n_in, (torch.bfloat16,))
+    shifted = torch.zeros(down.numel() + 1, dtype=down.dtype, device="cuda")[1:].view(down.shape)
+    shifted.copy_(down)
+    up = up.cuda()
+    assert shifted.data_ptr() % 4 == 2 and shifted.is_contiguous()
+    res = torch.zeros((n_out, n_in), dtype=torch.bfloat16, device="cuda")
+    rc = native.lib().wf_dequant_lora(None, 0, 0, 0, BF16, up.data_ptr(), BF16, shifted.data_ptr(), BF16, 16, s,
+                                      res.data_ptr(), n_out, n_in, native.stream_of(res.device))
+    assert rc == native.EUNSUPPORTED
+    y = gd.dequantize_lora(torch.from_numpy(raw).cuda(), 8, (n_out, n_in), None, torch.bfloat16, [(up, shifted, s)])
+    torch.cuda.synchronize()
+    ok, where = _same(_bits(y, BF16), _expected(raw, 8, F16, BF16, n_out, n_in, [(up, down, s)]), BF16)
+    assert ok, where
