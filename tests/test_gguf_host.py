@@ -209,3 +209,32 @@ def test_lora_route_by_rank_and_dtype(gd, monkeypatch, up, down, rank, kernel):
     assert gd._add_in_kernel(*args) is kernel
     assert gd._add_in_kernel(*args) or gd._add_difference(*args)
     assert calls.names == (["wf_dequant_lora"] * 2 if kernel else ["wf_dequant_add"])
+
+
+class _Scaled(torch.Tensor):
+    """A tensor that holds its values in another form (as a quantised one does): they appear where it is cast."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        if func is torch.Tensor.to and torch.float32 in args:
+            return args[0].as_subclass(torch.Tensor).float() * 4.0
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+def test_lora_factors_that_are_not_plain_tensors(gd, monkeypatch):
+    # the kernel reads a factor's memory: a subclass, or a view with its sign pending, takes comfy's cast as before
+    calls, seen = _LoraCalls(), []
+    monkeypatch.setattr(gd._native, "lib", lambda: calls)
+    mm = torch.mm
+    monkeypatch.setattr(torch, "mm", lambda a, b: seen.append((a, b)) or mm(a, b))
+    res = torch.zeros((8, 32), dtype=torch.float32)
+    up, down = torch.ones((8, 4)).as_subclass(_Scaled), torch.ones((4, 32))
+    for a, b, value in ((up, down, 4.0), (torch._neg_view(torch.ones((8, 4))), down, -1.0),
+                        (torch.nn.Parameter(torch.ones((8, 4)), requires_grad=False), down, None)):
+        del calls.names[:], seen[:]
+        args = ((None, 0, 0, 0), a, b, 1.0, res, "0", None)
+        assert gd._add_in_kernel(*args) or gd._add_difference(*args)
+        if value is None:
+            assert calls.names == ["wf_dequant_lora"]
+        else:
+            assert calls.names == ["wf_dequant_add"] and bool((seen[0][0] == value).all())
