@@ -926,7 +926,7 @@ __global__ __launch_bounds__(64 * kSpWaves) void gemm_gguf_splitk(const uint16_t
 // c ^ (r & 15) (the 16 rows of a fragment read fall in 16 different bank groups). The weight's raw bytes of the next
 // super-block load into the second of two register sets meanwhile, and each lane dequantises into its B fragments
 // as in the few-rows kernel; A fragments come from LDS.
-// K is split into S slices only as far as needed to give the chip 256 workgroups: with S > 1 each slice writes its
+// K is split into S slices by panel_plan (256 to 768 workgroups): with S > 1 each slice writes its
 // float32 partial sums (part[s][m][n]) and gguf_panel_sum adds them in slice order (deterministic), adds the bias
 // and rounds to bf16.
 constexpr int kPnWaves = 4;
@@ -1407,11 +1407,7 @@ struct PanelPlan {
 // Modelled ns of the panel form in s slices of ks super-blocks over `tiles` panels: a super-block costs its dequantisation
 // and, per 16 activation rows, its MFMAs; two workgroups share a CU in 1.58 times the time of one, three take 2.5 and
 // four 2.9 times; each slice's partial sums pass through memory once each way. Fitted to 432 measurements (Q4_K, Q6_K,
-// Q8_0; the Wan shapes and 2048 x 2048 at 40-400 rows, cold weights, MI355X; 6 % rms). Aiming for 256 workgroups (512
-// above 384 rows and for Q6_K up to 128) leaves a few CUs with one more than the others. The plan aims elsewhere where
-// that is modelled 8 % faster and slices keep three super-blocks (two were slower than modelled): 7 % on average over
-// those measurements, none slower: Q4_K 5120 x 5120 at 256 rows 33.2 against 37.3 us, Q6_K 5120 x 13824 at 300 rows 127
-// against 157, Q8_0 5120 x 13824 at 256 rows 92 against 124.
+// Q8_0; the Wan shapes and 2048 x 2048 at 40-400 rows, cold weights, MID float16, MI355X; 6 % rms).
 static int64_t panel_time(int64_t tiles, int64_t s, int64_t ks, int mt, int64_t outputs, int qtype) {
     const int64_t block = qtype == 14 ? 2252 + 368 * mt : qtype == 8 ? 2324 + 101 * mt : 1371 + 194 * mt;
     const int64_t turns = (tiles * s + 255) / 256;
@@ -1432,9 +1428,7 @@ static PanelPlan panel_plan(int64_t M, int64_t N, int64_t K, int64_t max_part, i
     // at 140 rows Q4_K 30.6 against 35.8 us, Q6_K 49.0 against 55.5). Q6_K's 48-row panels lost to 64-row ones (0.98)
     // and its 80-row ones to 96-row ones (13824 x 5120 at 77 rows 69.3 against 59.7 us).
     const int need = (int)((M + 16 * p.mti - 1) / (16 * p.mti));
-    // (the slices go by this height for every MID: the workspace query knows no MID)
-    const int height = qtype == 14 && (need == 3 || need == 5) ? need + 1 : std::max(2, need);
-    if (mid_dt == WF_F16) p.mt = height;
+    if (mid_dt == WF_F16) p.mt = qtype == 14 && (need == 3 || need == 5) ? need + 1 : std::max(2, need);
     p.nt = (int)((N + kPnRows - 1) / kPnRows);
     const int nsb = (int)(K / 256);
     const int64_t tiles = (int64_t)p.nt * p.mti;
@@ -1444,12 +1438,28 @@ static PanelPlan panel_plan(int64_t M, int64_t N, int64_t K, int64_t max_part, i
         const int ks = (nsb + s - 1) / s;
         return std::make_pair((nsb + ks - 1) / ks, ks);
     };
+    // Aiming for 256 workgroups (512 above 384 rows and for Q6_K up to 128) leaves a few CUs with one more than the others.
+    // The plan aims elsewhere where that is modelled 8 % faster (Q8_0 12 %), for MID float16 alone (the model's: with MID
+    // bfloat16 it cost 1424 x 10752 Q5_K at 488 rows 55 us against 47). Left as they are, since they measured slower than
+    // modelled: slices of under four super-blocks (Q4_K 3252 x 9472 at 23 rows 0.87 times as fast; three will do for Q4_K
+    // and Q5_K from an aim well over one workgroup a CU: Q5_K 3072 x 3072 at 512 rows 29.6 against 35.3 us), Q6_K and Q8_0
+    // a little over 512 workgroups (Q6_K 7248 x 6400 at 34 rows 0.81, Q8_0 1248 x 9472 at 471 rows 0.85), and two to three
+    // workgroups a CU for an aim just over one (Q4_K 12166 x 10240 at 119 rows 0.92). Over 345 random shapes that the model
+    // alone would move 1.13 times as fast, 9 of them 2-10 % slower: Q4_K 5120 x 5120 at 256 rows 33.2 against 37.3 us, Q6_K
+    // 5120 x 13824 at 300 rows 127 against 157, Q8_0 5120 x 13824 at 256 rows 92 against 124.
     std::tie(p.s, p.ks) = slices(M > 384 || (qtype == 14 && M <= 128) ? 512 : 256);
-    int64_t best = panel_time(tiles, p.s, p.ks, height, M * N, qtype) * 92 / 100;
-    for (int64_t target : {384, 512, 768}) {
-        const auto [s, ks] = slices(target);
-        const int64_t t = panel_time(tiles, s, ks, height, M * N, qtype);
-        if (ks >= 3 && t < best) { best = t; p.s = s; p.ks = ks; }
+    const int64_t held = tiles * p.s;
+    const int fewest = held > 320 && (qtype == 12 || qtype == 13) ? 3 : 4;
+    if (mid_dt == WF_F16 && !((qtype == 8 || qtype == 14) && held > 512 && held <= 600)) {
+        int64_t best = panel_time(tiles, p.s, p.ks, p.mt, M * N, qtype) * (qtype == 8 ? 88 : 92) / 100;
+        for (int64_t target : {384, 512, 768}) {
+            const auto [s, ks] = slices(target);
+            const int64_t t = panel_time(tiles, s, ks, p.mt, M * N, qtype), groups = tiles * s;
+            if (ks < fewest || t >= best || (held <= 320 && groups > 512 && groups <= 768)) continue;
+            best = t;
+            p.s = s;
+            p.ks = ks;
+        }
     }
     p.part_bytes = p.s > 1 ? (int64_t)p.s * M * N * 4 : 0;
     return p;
@@ -1567,12 +1577,12 @@ extern "C" int wf_linear_gguf_workspace(int64_t M, int64_t N, int64_t K, int64_t
     if (!bytes) { set_error("wf_linear_gguf_workspace: null out-pointer"); return WF_EINVAL; }
     *bytes = 0;
     if (M < 0 || N < 0 || K <= 0 || K % 256) { set_error("wf_linear_gguf_workspace: M, N, K"); return WF_EINVAL; }
-    // the format is not known here: the largest need over them (Q6_K's panels take more slices up to 128 rows)
+    // format and MID are not known here: the largest need over them
     if (split_takes(M, N, K)) *bytes = split_plan(M, N, K).bytes();
     else if (panel_takes_ws(M, N, K)) {
-        const int64_t part = std::max({panel_plan(M, N, K, INT64_MAX, 12, WF_F16).part_bytes,
-                                       panel_plan(M, N, K, INT64_MAX, 14, WF_F16).part_bytes,
-                                       panel_plan(M, N, K, INT64_MAX, 8, WF_F16).part_bytes});
+        int64_t part = 0;
+        for (int qtype : {12, 14, 8})
+            for (int mid : {WF_F16, WF_BF16}) part = std::max(part, panel_plan(M, N, K, INT64_MAX, qtype, mid).part_bytes);
         if (part > 0) *bytes = kSplitCounterBytes + part;   // the split form's counters stay untouched
     }
     return WF_OK;

@@ -4,6 +4,8 @@ Reference: a float64 GEMM of the same bf16 activations with the oracle's bit-exa
 reference path: dequantize, then F.linear in bf16). The tolerance is the task's bound for bf16 GEMMs, max relative error
 <= 1e-2 (max |y - ref| / max |ref|); each element is also held to |y - ref| <= 2^-8 |ref| + 1e-3 max |ref|, which
 only a correct weight meets (float32 accumulation order and the final bf16 rounding stay well inside it)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -478,3 +480,22 @@ def test_panel_heights(native, qtype):
         y, _, need = fused_ws(native, x[:M].cuda(), rd, qtype, N)
         assert need > 0
         check(y, x[:M], w)
+
+
+@pytest.mark.parametrize("qtype", [12, 13, 14, 8])
+@pytest.mark.parametrize("M,N,K", [(488, 1424, 10752), (300, 1300, 6656), (63, 2090, 4096), (20, 3252, 9472)])
+def test_panel_slices_of_every_mid_fit_the_workspace(native, qtype, M, N, K):
+    # the slices depend on MID (float16 alone goes by the model), the workspace query knows none: every MID's partial sums
+    # stay inside the bytes it asks for, and the sums are right
+    need = ctypes.c_int64()
+    assert native.lib().wf_linear_gguf_workspace(M, N, K, ctypes.byref(need)) == 0 and need.value > 0
+    raw = encode.random_blocks(qtype, nblocks(qtype, N, K), seed=qtype, family="normal")
+    rd = torch.from_numpy(raw).cuda()
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).cuda()
+    held = torch.zeros(need.value + 4096, dtype=torch.uint8, device="cuda")
+    held[need.value:] = 0x5A
+    for mid in range(3):
+        print(f"case panel slices qtype={qtype} mid={mid} {M}x{N}x{K}", flush=True)
+        y, _, _ = fused_ws(native, x, rd, qtype, N, mid=mid, ws=held[:need.value])
+        check_gpu(y, x, weight_bf16(raw, qtype, mid, N, K))
+        assert bool((held[need.value:] == 0x5A).all())
