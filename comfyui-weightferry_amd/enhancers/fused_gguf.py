@@ -129,14 +129,16 @@ def prefer_fused(rows, qtype, n_out, k):
     return rows <= limit
 
 
-# Q5_K at 385-512 rows, outputs no wider than K: with the panel form's K slices chosen by time the fused kernel beats the
-# two-step flow there too (us, cold weights, MI355X): 5120 x 5120 51.6 / 54.3 against 60.9 / 61.6 at 385 / 512 rows,
-# 5120 x 13824 113.7 against 142.4 and 2048 x 2048 23.1 against 28.6 at 512; the closest, 8192 x 9216, 114.3 / 128.6
-# against 119.5 / 123.7 at 400 / 512. Q6_K above 256 rows stays slower on most shapes (5120 x 5120 at 300 rows 52.7
-# against 47.4).
-def prefer_slices(rows, qtype, n_out, k):
+# Q5_K at 385-512 rows, outputs of whole 128-row panels up to 5120 wide and no wider than K: with the panel form's K slices
+# the fused kernel beats the two-step flow there too (us, MI355X): 5120 x 5120 47 / 52 against 57 / 61 at 385 / 512 rows,
+# 5120 x 13824 113 against 139 and 2048 x 2048 22.8 against 28.3 at 512. Elsewhere it does not: wider outputs (6144 x 6144
+# 74.8 against 69.6 at 512 rows, 9216 x 9216 147 against 134, 8192 x 8192 105.5 against 104.2), partial panels (1726 x 12800
+# 0.84 times as fast at 471 rows), MID bfloat16 (5120 x 5120 61.7 against 57.7 at 385 rows) and float32 (3072 x 3072 0.9 times
+# as fast). Q6_K above 256 rows stays slower on most shapes (5120 x 5120 at 300 rows 52.7 against 47.4).
+def prefer_slices(rows, qtype, n_out, k, mid_dtype=None):
     """mode "auto" beyond ``prefer_fused``: True where the panel form in K slices is the faster one."""
-    return qtype == 13 and PANEL_ROWS[13] < rows <= 512 and n_out <= k
+    return (qtype == 13 and PANEL_ROWS[13] < rows <= 512 and n_out <= min(k, 5120) and n_out % 128 == 0
+            and mid_dtype in (None, torch.float16))
 
 
 # The two-step flow's GEMM: the library's wf_linear_bf16 (whole 128-byte lines through two LDS stage buffers, 256 x 320
@@ -184,7 +186,7 @@ def linear(x, data, qtype, oshape, bias=None, mid_dtype=None, mode="auto"):
     rows = x.numel() // max(1, x.shape[-1]) if x.dim() else 0
     if mode == "auto":
         n_out, k = oshape[0], oshape[1]
-        fused = prefer_fused(rows, qtype, n_out, k) or prefer_slices(rows, qtype, n_out, k)
+        fused = prefer_fused(rows, qtype, n_out, k) or prefer_slices(rows, qtype, n_out, k, mid_dtype)
         mode = "fused" if fused else "dequant"
     if mode == "fused":
         y = fused_linear(x, data, qtype, oshape, bias, mid_dtype)

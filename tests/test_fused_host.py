@@ -58,6 +58,15 @@ def test_prefer_slices_rule():
     assert not fg.prefer_slices(384, 13, 5120, 5120) and not fg.prefer_slices(513, 13, 5120, 5120)
 
 
+def test_prefer_slices_keeps_to_what_measured_faster():
+    for rows in (385, 512):
+        for n_out, k in ((8192, 9216), (8192, 8192), (6144, 6144), (9216, 9216), (1726, 12800), (5088, 5120)):
+            assert not fg.prefer_slices(rows, 13, n_out, k)
+        assert fg.prefer_slices(rows, 13, 2048, 8192, torch.float16)
+        for mid in (torch.bfloat16, torch.float32):
+            assert not fg.prefer_slices(rows, 13, 5120, 5120, mid)
+
+
 def test_auto_routes_by_rows(monkeypatch):
     calls = []
 
