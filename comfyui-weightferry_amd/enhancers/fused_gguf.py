@@ -141,6 +141,19 @@ def prefer_slices(rows, qtype, n_out, k, mid_dtype=None):
             and mid_dtype in (None, torch.float16))
 
 
+def _only_product(x, bias):
+    """Whether torch.nn.functional.linear on ``x`` would do no more than the product: it records gradients, carries
+    forward-mode tangents, and goes through transforms (vmap) and tensor subclasses; the kernels read memory."""
+    for t in (x,) if bias is None else (x, bias):
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or (t.requires_grad and torch.is_grad_enabled()):
+            return False
+        if torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+        if torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+            return False
+    return True
+
+
 # The two-step flow's GEMM: the library's wf_linear_bf16 (whole 128-byte lines through two LDS stage buffers, 256 x 320
 # tiles at these sizes) against hipBLASLt's (torch.nn.functional.linear), ms per Wan-14B shape on MI355X:
 #   4096 rows: 5120 x 5120 0.165 against 0.176, 5120 x 13824 0.432 against 0.449, 13824 x 5120 0.459 against 0.404
@@ -186,7 +199,8 @@ def linear(x, data, qtype, oshape, bias=None, mid_dtype=None, mode="auto"):
     rows = x.numel() // max(1, x.shape[-1]) if x.dim() else 0
     if mode == "auto":
         n_out, k = oshape[0], oshape[1]
-        fused = prefer_fused(rows, qtype, n_out, k) or prefer_slices(rows, qtype, n_out, k, mid_dtype)
+        fused = prefer_fused(rows, qtype, n_out, k) or (prefer_slices(rows, qtype, n_out, k, mid_dtype)
+                                                        and _only_product(x, bias))
         mode = "fused" if fused else "dequant"
     if mode == "fused":
         y = fused_linear(x, data, qtype, oshape, bias, mid_dtype)

@@ -128,3 +128,35 @@ def test_two_step_routes_its_gemm(monkeypatch):
     fg.linear(torch.zeros(1, 4096, 256, dtype=torch.bfloat16), data, 12, (5120, 256), mode="dequant")
     fg.linear(torch.zeros(1, 2048, 256, dtype=torch.bfloat16), data, 12, (5120, 256), mode="dequant")
     assert calls == ["hand", "torch"]
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def test_rows_that_take_slices_keep_what_the_two_step_flow_gives_beside_the_product(monkeypatch):
+    # Q5_K at 385-512 rows went through torch's linear, which records gradients and goes through transforms and subclasses:
+    # where any of these is there it still does
+    calls = []
+    monkeypatch.setattr(fg, "fused_linear",
+                        lambda x, data, q, oshape, *a: calls.append("fused") or x.new_zeros(*x.shape[:-1], oshape[0]))
+    monkeypatch.setattr(fg.gguf_dequant, "dequantize", lambda d, q, oshape, mid=None, out=None:
+                        calls.append("dequant") or torch.ones(oshape, dtype=out))
+    data, weight = torch.zeros(16, dtype=torch.uint8), (128, 256)
+
+    def route(x, bias=None):
+        del calls[:]
+        return fg.linear(x, data, 13, weight, bias), calls[0]
+    x, b = torch.ones(400, 256), torch.zeros(128)
+    assert route(x)[1] == "fused" and route(x, b)[1] == "fused"
+    y, how = route(x.clone().requires_grad_())
+    assert how == "dequant" and y.requires_grad
+    assert route(x, b.clone().requires_grad_())[1] == "dequant"
+    with torch.no_grad():
+        assert route(x.clone().requires_grad_())[1] == "fused"
+    assert route(x.as_subclass(_Sub))[1] == "dequant"
+    with torch.autograd.forward_ad.dual_level():
+        y, how = route(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+        assert how == "dequant" and torch.autograd.forward_ad.unpack_dual(y).tangent is not None
+    out = torch.func.vmap(lambda v: fg.linear(v, data, 13, weight))(torch.ones(3, 400, 256))
+    assert calls[-1] == "dequant" and out.shape == (3, 400, 128)

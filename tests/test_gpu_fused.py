@@ -499,3 +499,20 @@ def test_panel_slices_of_every_mid_fit_the_workspace(native, qtype, M, N, K):
         y, _, _ = fused_ws(native, x, rd, qtype, N, mid=mid, ws=held[:need.value])
         check_gpu(y, x, weight_bf16(raw, qtype, mid, N, K))
         assert bool((held[need.value:] == 0x5A).all())
+
+
+def test_gradients_at_the_rows_that_take_slices(native):
+    # Q5_K at 385-512 rows: a gradient that is asked for still comes back (the two-step flow), and without one the fused
+    # kernel runs; both give the product
+    M, N, K = 448, 256, 1024
+    fg = sub("enhancers.fused_gguf")
+    raw = encode.random_blocks(13, nblocks(13, N, K), seed=3, family="normal")
+    w, rd = weight_bf16(raw, 13, 0, N, K), torch.from_numpy(raw).cuda()
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).cuda().requires_grad_()
+    y = fg.linear(x, rd, 13, (N, K))
+    g = torch.randn((M, N), generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).cuda()
+    y.backward(g)
+    check(y.detach(), x.detach(), w)
+    check(x.grad, g, w.T.contiguous())
+    with torch.no_grad():
+        check(fg.linear(x, rd, 13, (N, K)), x.detach(), w)
