@@ -25,11 +25,14 @@ _needs = {}                  # (rows, n_out, k) -> the workspace bytes wf_linear
 def _workspace(device, stream, nbytes):
     """The split-K workspace of this device and stream, at least ``nbytes``: allocated zeroed once (its counters
     must be zero on entry, and every call leaves them zero) and grown when a larger product needs more. Calls on one
-    stream are ordered, so they can share it."""
+    stream are ordered, so they can share it. None when there is no memory for it (the one held stays)."""
     key = (device.index, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+        try:
+            ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            return None
         _workspaces[key] = ws
     return ws
 
@@ -56,7 +59,8 @@ def _launch(x2, rows, raw, raw_bytes, q, n_out, k, b, y, mid, dev):
         need = _workspace_bytes(rows, n_out, k)
     if need:                        # the split or panel form (K in slices) with its workspace
         ws = _workspace(dev, stream, need)
-        return _native.lib().wf_linear_gguf_ws(*args, ws.data_ptr(), ws.numel(), stream)
+        if ws is not None:
+            return _native.lib().wf_linear_gguf_ws(*args, ws.data_ptr(), ws.numel(), stream)
     return _native.lib().wf_linear_gguf(*args, stream)
 
 

@@ -160,3 +160,27 @@ def test_rows_that_take_slices_keep_what_the_two_step_flow_gives_beside_the_prod
         assert how == "dequant" and torch.autograd.forward_ad.unpack_dual(y).tangent is not None
     out = torch.func.vmap(lambda v: fg.linear(v, data, 13, weight))(torch.ones(3, 400, 256))
     assert calls[-1] == "dequant" and out.shape == (3, 400, 128)
+
+
+def test_no_memory_for_the_workspace_runs_without_it(monkeypatch):
+    # a card filled by resident weights: the call needs no workspace, it is only faster with one
+    names = []
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *a: names.append(name) or 0
+
+    def zeros(*a, **kw):
+        raise torch.OutOfMemoryError("no memory")
+    monkeypatch.setattr(fg._native, "lib", lambda: Lib())
+    monkeypatch.setattr(fg._native, "stream_of", lambda dev: 7)
+    monkeypatch.setattr(fg, "_workspace_bytes", lambda rows, n_out, k: 1 << 24)
+    monkeypatch.setattr(fg, "_needs", {})
+    monkeypatch.setattr(fg, "_workspaces", {})
+    x, raw = torch.zeros(100, 256, dtype=torch.bfloat16), torch.zeros(64 * 144, dtype=torch.uint8)
+    y = torch.zeros(100, 64, dtype=torch.bfloat16)
+    args = (x, 100, raw, raw.numel(), 12, 64, 256, None, y, 0, torch.device("cpu"))
+    assert fg._launch(*args) == 0 and names == ["wf_linear_gguf_ws"]
+    monkeypatch.setattr(fg, "_workspaces", {})
+    monkeypatch.setattr(torch, "zeros", zeros)
+    assert fg._launch(*args) == 0 and names[1:] == ["wf_linear_gguf"] and fg._workspaces == {}
