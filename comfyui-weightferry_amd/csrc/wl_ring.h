@@ -39,10 +39,11 @@ struct WlShape {
 // The order of a K step is pinned: behind each MFMA the next K step's fragment reads that fall to it, and in the last
 // step the next stage's loads, one by one, each followed by a scheduling barrier. Left to the compiler the reads come
 // in a burst before the MFMAs and the loads in one behind them; spread, they pass under the matrix unit. Measured on
-// MI355X (us): int8 5152 x 2048 x 8192 84.1 against 87.4, 5152 x 8192 x 2048 95.5 against 97.9, 16384 x 5120 x 5120
-// 359.0 against 361.6; bf16 4096 x 5120 x 5120 159.3 against 161.8, 4096 x 13824 x 5120 454.5 against 457.0. What is
-// left is the loads' and the reads' own cost: bf16 16384 x 5120 x 5120 takes 636, 551 without the loads, 529 without
-// the reads, 419 with neither.
+// MI355X, in turn on random operands (us): int8 5152 x 8192 x 2048 92.6 against 95.3, 4096 x 5120 x 5120 89.3 against 90.0;
+// bf16 4096 x 5120 x 5120 159.3 against 161.7, 4096 x 13824 x 5120 454.1 against 458.6. At 16384 rows, under the power
+// limit, the runs resolve no difference (int8 16384 x 5120 x 5120 362 against 364, 16384 x 13824 x 5120 982 against 982).
+// What is left is the loads' and the reads' own cost: bf16 16384 x 5120 x 5120 takes 636, 551 without the loads, 529
+// without the reads, 419 with neither.
 template <typename S, typename Acc, typename Mma>
 __device__ __forceinline__ void wl_mainloop(__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, uint32_t KB, int s0,
                                             int nk, int wave, int lane, wl_frag* sb0, wl_frag* sb1,

@@ -159,12 +159,11 @@ def _only_product(x, bias):
 
 
 # The two-step flow's GEMM: the library's wf_linear_bf16 (whole 128-byte lines through two LDS stage buffers, 256 x 320
-# tiles at these sizes) against hipBLASLt's (torch.nn.functional.linear), ms per Wan-14B shape on MI355X:
-#   4096 rows: 5120 x 5120 0.165 against 0.176, 5120 x 13824 0.432 against 0.449, 13824 x 5120 0.459 against 0.404
-#              (704 tiles: 2.75 rounds of 256 workgroups) -- the block's six linears 1.546 against 1.549;
-#   2048 rows and fewer: 0.104-0.114 against 0.095 (5120 x 5120) -- 128 or fewer 256 x 320 tiles leave CUs idle;
-#   16384 rows: 0.640 against 0.562 (5120 x 5120), 6.07 against 5.47 per block -- hipBLASLt's stream-K kernel keeps
-#              its MFMA 83 % busy against 73 % here.
+# tiles at these sizes) against hipBLASLt's (torch.nn.functional.linear), ms per Wan-14B shape on MI355X, in turn:
+#   4096 rows: 5120 x 5120 0.159 against 0.179, 5120 x 13824 0.418 against 0.451, 13824 x 5120 0.454 against 0.467
+#              (704 tiles: 2.75 rounds of 256 workgroups; the closest of the range); 8192 rows 5120 x 5120 0.313 against 0.462;
+#   2048 rows: 13824 x 5120 0.259 against 0.244 (352 tiles, a short second round; inside the rule all the same);
+#   16384 rows: 5120 x 5120 0.635 against 0.607 -- hipBLASLt's stream-K kernel keeps its MFMA 83 % busy against 73 % here.
 # So wf_linear_bf16 takes the products whose 256 x 320 tiling gives one to three rounds of 256 workgroups.
 HAND_GEMM_TILES = (256, 768)
 

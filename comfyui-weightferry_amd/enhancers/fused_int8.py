@@ -63,7 +63,8 @@ def quantise_rows(x_2d, mode):
 # takes less GPU time than its call takes the thread gains nothing and is that much slower, so it runs whole: below
 # _LEAST_NS for int8_linear (its call 24 us whole, 29 in slices on MI355X: 2048 x 2048 at 4-150 rows 24.2 against 29.4 us,
 # 5120 x 5120 at 16 rows 32.6 against 29.2), below _BLOCK_LEAST_NS for a layer of a block, whose eligibility checks take
-# longer (a QKV of three layers 315 us whole, 331 in slices at 2048 and 4096 wide, 32-256 rows).
+# longer (a QKV of three layers, 2048 and 4096 wide at 64-256 rows: 95 us whole, 108-110 in slices with ComfyUI's modules
+# importable, 315 and 331 without).
 _LEAST_NS, _BLOCK_LEAST_NS = 26_000, 100_000
 _plans = {}                  # (m, n, k) -> (the bytes K slices need, 0: none; the modelled ns without them)
 
