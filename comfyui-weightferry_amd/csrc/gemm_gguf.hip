@@ -1404,15 +1404,23 @@ struct PanelPlan {
     int64_t part_bytes;
 };
 
-// Modelled ns of the panel form in s slices of ks super-blocks over `tiles` panels: a super-block costs its dequantisation
-// and, per 16 activation rows, its MFMAs; two workgroups share a CU in 1.58 times the time of one, three take 2.5 and
-// four 2.9 times; each slice's partial sums pass through memory once each way. Fitted to 432 measurements (Q4_K, Q6_K,
-// Q8_0; the Wan shapes and 2048 x 2048 at 40-400 rows, cold weights, MID float16, MI355X; 6 % rms).
-static int64_t panel_time(int64_t tiles, int64_t s, int64_t ks, int mt, int64_t outputs, int qtype) {
+// Modelled ns of the panel form in s slices of ks super-blocks (the last one of what is left of nsb) over `tiles` panels: a
+// super-block costs its dequantisation and, per 16 activation rows, its MFMAs; two workgroups share a CU in 1.58 times the
+// time of one, three take 2.5 and four 2.9 times; each slice's partial sums pass through memory once each way. Fitted to
+// 432 measurements (Q4_K, Q6_K, Q8_0; the Wan shapes and 2048 x 2048 at 40-400 rows, cold weights, MID float16, MI355X; 6 %
+// rms). The last slices start last: where they alone make up a CU's second (third, ...) turn, that CU shares its time only
+// as long as they run. Without this, slices that divide K badly looked as slow as their longest, and leaving them cost up to
+// 19 % (Q6_K 7248 x 6400 at 34 rows).
+static int64_t panel_time(int64_t tiles, int64_t s, int64_t ks, int64_t nsb, int mt, int64_t outputs, int qtype) {
     const int64_t block = qtype == 14 ? 2252 + 368 * mt : qtype == 8 ? 2324 + 101 * mt : 1371 + 194 * mt;
-    const int64_t turns = (tiles * s + 255) / 256;
-    const int64_t share = turns <= 1 ? 1000 : turns == 2 ? 1577 : turns == 3 ? 2497 : 732 * turns;
-    return ks * block * share / 1000 + (s > 1 ? s * outputs * 1542 / 1000000 : 0);
+    auto share = [](int64_t turns) -> int64_t {
+        return turns <= 1 ? 1000 : turns == 2 ? 1577 : turns == 3 ? 2497 : 732 * turns;
+    };
+    const int64_t turns = (tiles * s + 255) / 256, last = nsb - (s - 1) * ks;
+    const bool short_end = turns > 1 && tiles * s - 256 * (turns - 1) <= tiles;
+    const int64_t shared = short_end ? last : ks;
+    return (shared * share(turns) + (ks - shared) * share(turns - 1)) * block / 1000 +
+           (s > 1 ? s * outputs * 1542 / 1000000 : 0);
 }
 
 static PanelPlan panel_plan(int64_t M, int64_t N, int64_t K, int64_t max_part, int qtype, int mid_dt) {
@@ -1439,23 +1447,17 @@ static PanelPlan panel_plan(int64_t M, int64_t N, int64_t K, int64_t max_part, i
         return std::make_pair((nsb + ks - 1) / ks, ks);
     };
     // Aiming for 256 workgroups (512 above 384 rows and for Q6_K up to 128) leaves a few CUs with one more than the others.
-    // The plan aims elsewhere where that is modelled 8 % faster (Q8_0 12 %), for MID float16 alone (the model's: with MID
-    // bfloat16 it cost 1424 x 10752 Q5_K at 488 rows 55 us against 47). Left as they are, since they measured slower than
-    // modelled: slices of under four super-blocks (Q4_K 3252 x 9472 at 23 rows 0.87 times as fast; three will do for Q4_K
-    // and Q5_K from an aim well over one workgroup a CU: Q5_K 3072 x 3072 at 512 rows 29.6 against 35.3 us), Q6_K and Q8_0
-    // a little over 512 workgroups (Q6_K 7248 x 6400 at 34 rows 0.81, Q8_0 1248 x 9472 at 471 rows 0.85), and two to three
-    // workgroups a CU for an aim just over one (Q4_K 12166 x 10240 at 119 rows 0.92). Over 345 random shapes that the model
-    // alone would move 1.13 times as fast, 9 of them 2-10 % slower: Q4_K 5120 x 5120 at 256 rows 33.2 against 37.3 us, Q6_K
-    // 5120 x 13824 at 300 rows 127 against 157, Q8_0 5120 x 13824 at 256 rows 92 against 124.
+    // The plan aims elsewhere where that is modelled 8 % faster (Q8_0 12 %) and slices keep three super-blocks, for MID
+    // float16 alone (the model's: with MID bfloat16 it cost 1424 x 10752 Q5_K at 488 rows 55 us against 47). Over 665 random
+    // shapes that a cruder model would move 1.16 times as fast, 10 of them 2-9 % slower: Q4_K 5120 x 5120 at 256 rows 33.2
+    // against 37.3 us, Q6_K 5120 x 13824 at 300 rows 127 against 157, Q8_0 5120 x 13824 at 256 rows 92 against 124.
     std::tie(p.s, p.ks) = slices(M > 384 || (qtype == 14 && M <= 128) ? 512 : 256);
-    const int64_t held = tiles * p.s;
-    const int fewest = held > 320 && (qtype == 12 || qtype == 13) ? 3 : 4;
-    if (mid_dt == WF_F16 && !((qtype == 8 || qtype == 14) && held > 512 && held <= 600)) {
-        int64_t best = panel_time(tiles, p.s, p.ks, p.mt, M * N, qtype) * (qtype == 8 ? 88 : 92) / 100;
+    if (mid_dt == WF_F16) {
+        int64_t best = panel_time(tiles, p.s, p.ks, nsb, p.mt, M * N, qtype) * (qtype == 8 ? 88 : 92) / 100;
         for (int64_t target : {384, 512, 768}) {
             const auto [s, ks] = slices(target);
-            const int64_t t = panel_time(tiles, s, ks, p.mt, M * N, qtype), groups = tiles * s;
-            if (ks < fewest || t >= best || (held <= 320 && groups > 512 && groups <= 768)) continue;
+            const int64_t t = panel_time(tiles, s, ks, nsb, p.mt, M * N, qtype);
+            if (ks < 3 || t >= best) continue;
             best = t;
             p.s = s;
             p.ks = ks;
